@@ -86,29 +86,21 @@ __global__ void __launch_bounds__(256) k_setup_edges(DevMesh M, DevGeomOut G) {
 
 // ReconstructFullWetCell (src/MUSCLObject.cpp:38-84): the limited plane of
 // cell (vertices p0..p2, flags fl, level w, centroid cx, cy) from its
-// neighbours' levels wn, records rn and ids jn (a partially wet neighbour's
-// full record is read from M.crec).
+// neighbours' levels wn and records rn, none of them dry; a partially wet
+// neighbour (pw) has its pass-1 level in its record's zmx.
 template <bool HEAD_GRAD>
-__device__ __forceinline__ void fullwet_plane(const DevMesh& M, const V3& p0, const V3& p1, const V3& p2,
-                                              uint32_t fl, double w, double cx, double cy, const double wn[3],
-                                              const NRec rn[3], const int jn[3], double& gx, double& gy) {
-  gx = 0.;
-  gy = 0.;
+__device__ __forceinline__ void fullwet_plane(const V3& p0, const V3& p1, const V3& p2, uint32_t fl, double w,
+                                              double cx, double cy, const double wn[3], const NRec rn[3],
+                                              const bool pw[3], double& gx, double& gy) {
   V3 pts[3];
   V3 E[3];
-  bool any_dry = false;
 #pragma unroll
   for (int kk = 0; kk < 3; ++kk) {
     E[kk] = edge_mid(p0, p1, p2, fl, kk);
-    const double wj = wn[kk], bcj = rn[kk].bc;
-    if (rn[kk].zmx < wj) {  // interior full-wet neighbour (zmx = +inf on boundary cells)
-      pts[kk] = {rn[kk].cx, rn[kk].cy, HEAD_GRAD ? bcj : wj};
-    } else if (!is_wet(wj - bcj)) {
-      any_dry = true;
-      pts[kk] = {0., 0., 0.};
+    if (!pw[kk]) {  // interior full-wet neighbour
+      pts[kk] = {rn[kk].cx, rn[kk].cy, HEAD_GRAD ? rn[kk].bc : wn[kk]};
     } else {
-      const CellRec rj = M.crec[jn[kk]];  // partially wet neighbour: the full record
-      double w0j = partwet1_w(rj.zmin, rj.zmin, rj.zmax, bcj, wj);
+      const double w0j = rn[kk].zmx;
       double dx = E[kk].x - rn[kk].cx, dy = E[kk].y - rn[kk].cy;
       double a = w0j + (0. * dx + 0. * dy);
       if (!((a - E[kk].z) >= 0)) a = E[kk].z;
@@ -116,7 +108,6 @@ __device__ __forceinline__ void fullwet_plane(const DevMesh& M, const V3& p0, co
       pts[kk] = {E[kk].x, E[kk].y, HEAD_GRAD ? E[kk].z : val};
     }
   }
-  if (any_dry) return;
   gradient(pts[0], pts[1], pts[2], gx, gy);
   // vertex positivity (src/MUSCLObject.cpp:66-72)
   const double c23 = 1. - 1. / 3., c13 = -1. / 3.;
@@ -150,16 +141,42 @@ __device__ __forceinline__ void fullwet_plane(const DevMesh& M, const V3& p0, co
 // SpaceDisc::ComputeInterfaceValues pass 1 (src/SpaceDisc.cpp:37-45) with
 // ReconstructDryCell / ReconstructPartWetCell1 / ReconstructFullWetCell
 // (src/MUSCLObject.cpp:31-112).
+//
+// The levels of partially wet cells (PartWet1: a cube root or a bisection of
+// ~45 dependent cubic evaluations) are a serial chain of several us.  A wave
+// would run it up to four times in a row, for its partially wet cells and
+// then for each neighbour of its full-wet ones, with a few lanes active.  So
+// the workgroup lists the cells whose level its cells need, once each (its
+// own partially wet cells, whose neighbours in the workgroup share the
+// result, and the partially wet neighbours outside), and evaluates the list
+// one cell per lane: the chain is paid once.  Us per launch, before / now:
+// 35.0 / 10.8 (Thacker bowl, 1,600 cells), 25.0 / 10.4 (40,000), dam break
+// 28.7 / 13.5 (250k cells), 40 / 27.9 (1M), 100 / 92.5 (4M); without
+// partially wet cells 4.9 / 4.9 (62k).
 template <bool HEAD_GRAD, bool NT>
 __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W) {
   // The workgroup's 256 Morton-consecutive cells stage their level and the
   // part of their record a neighbour reads (NRec) in LDS; most neighbours
   // lie in the same workgroup and are read from there, the others from
-  // global memory.
-  __shared__ double s_w[kBlock];
-  __shared__ NRec s_r[kBlock];
+  // global memory.  The list of levels takes the same LDS afterwards: a
+  // cell asks for its own level or for up to three neighbours'.
+  struct Window {
+    double w[kBlock];
+    NRec r[kBlock];
+  };
+  struct Levels {
+    double lvl[3 * kBlock];
+    int cell[3 * kBlock];
+    int16_t own[kBlock];  // list entry of the workgroup's own cells, -1: the level is w
+  };
+  __shared__ union {
+    Window win;
+    Levels lev;
+  } sh;
+  __shared__ int s_n;
   const int64_t blk0 = M.c0 + (int64_t)logical_block() * kBlock;
   const int64_t i = blk0 + threadIdx.x;
+  const int tid = threadIdx.x;
   const bool live = i < M.c1;
   const int is = live ? (int)i : (int)M.c0;  // threads past the end read a valid cell
   // every load that does not need the LDS window is issued before the
@@ -185,40 +202,88 @@ __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W
       rn[kk] = M.nrec[j];
     }
   }
-  const V3 p0 = node(M, cvi.v0), p1 = node(M, cvi.v1), p2 = node(M, cvi.v2);
+  V3 p0 = node(M, cvi.v0), p1 = node(M, cvi.v1), p2 = node(M, cvi.v2);
   if (live) {
-    s_w[threadIdx.x] = w;
-    s_r[threadIdx.x] = ri;
+    sh.win.w[tid] = w;
+    sh.win.r[tid] = ri;
   }
+  if (tid == 0) s_n = 0;
   __syncthreads();
-  if (!live) return;
-  if (M.cinst && !M.bactive[M.cinst[i]]) return;  // finished ensemble member
+  // finished ensemble members are left alone
+  const bool on = live && !(M.cinst && !M.bactive[M.cinst[is]]);
 #pragma unroll
   for (int kk = 0; kk < 3; ++kk)
     if (inb[kk]) {
       const int64_t lj = jn[kk] - blk0;
-      wn[kk] = s_w[lj];
-      rn[kk] = s_r[lj];
+      wn[kk] = sh.win.w[lj];
+      rn[kk] = sh.win.r[lj];
     }
   const double bc = ri.bc;
   const double cx = ri.cx, cy = ri.cy;
-  double w0 = w, gx = 0., gy = 0.;
+  int8_t k = 0;
+  if (is_wet(w - bc)) k = ri.zmx < w ? 2 : 1;  // 1: a boundary cell (zmx = +inf) or a vertex at or above w
   double zmx = 0.;  // the highest vertex, read where pass 1 or 2 needs it
-  int8_t k;
-  if (!is_wet(w - bc)) {
-    k = 0;
+  if (on && k == 1) zmx = M.crec[is].zmax;
+  // the levels to evaluate: the cell's own and those of its partially wet
+  // neighbours outside the workgroup (those inside are their owners'); where
+  // the water stands above every vertex (wet boundary cells mostly) the level
+  // is w.  A neighbour's level takes the place of its record's zmx.  None
+  // where a dry neighbour leaves the plane out, none for HEAD's plane.
+  const bool own = on && k == 1 && !(w >= zmx);
+  bool nb[3] = {false, false, false}, out[3] = {false, false, false}, any_dry = false;
+  if (on && k == 2) {
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk) {
+      const bool full = rn[kk].zmx < wn[kk], wet = is_wet(wn[kk] - rn[kk].bc);
+      nb[kk] = !full && wet;
+      any_dry = any_dry || (!full && !wet);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk)
+      if (!HEAD_GRAD && nb[kk] && !any_dry) {
+        rn[kk].zmx = wn[kk];
+        out[kk] = !inb[kk] && !(wn[kk] >= M.crec[jn[kk]].zmax);
+      }
+  }
+  double w0 = w, gx = 0., gy = 0.;
+  if (__syncthreads_or(own || out[0] || out[1] || out[2])) {  // and every read of the window is done
+    int at[3] = {-1, -1, -1};
+    if (own) {
+      at[0] = atomicAdd(&s_n, 1);
+      sh.lev.cell[at[0]] = is;
+    }
+    sh.lev.own[tid] = (int16_t)at[0];
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk)
+      if (out[kk]) {
+        at[kk] = atomicAdd(&s_n, 1);
+        sh.lev.cell[at[kk]] = jn[kk];
+      }
+    __syncthreads();
+    const int n = s_n;
+    for (int q = tid; q < n; q += kBlock) {
+      // b13 = zmax, b23 = zmin enter partwet1_w only through max / min
+      const int j = sh.lev.cell[q];
+      const CellRec r = M.crec[j];
+      sh.lev.lvl[q] = partwet1_w(r.zmin, r.zmin, r.zmax, r.bc, S.w[S.at(j)]);
+    }
+    __syncthreads();
+    if (own) w0 = sh.lev.lvl[at[0]];
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk)
+      if (nb[kk] && !any_dry) {
+        const int q = inb[kk] ? sh.lev.own[jn[kk] - blk0] : at[kk];
+        if (q >= 0) rn[kk].zmx = sh.lev.lvl[q];
+      }
+  }
+  if (!on) return;
+  if (k == 0) {
     w0 = bc;
     gradient(p0, p1, p2, gx, gy);
-  } else if (!(ri.zmx < w)) {  // a boundary cell (zmx = +inf) or a vertex at or above w
-    k = 1;
-    // b13 = zmax, b23 = zmin enter partwet1_w only through max / min
-    const CellRec rf = M.crec[i];
-    zmx = rf.zmax;
-    w0 = partwet1_w(rf.zmin, rf.zmin, zmx, bc, w);
+  } else if (k == 1) {
     W.wrec1[i] = w0;
-  } else {
-    k = 2;
-    fullwet_plane<HEAD_GRAD>(M, p0, p1, p2, fl, w, cx, cy, wn, rn, jn, gx, gy);
+  } else if (!any_dry) {
+    fullwet_plane<HEAD_GRAD>(p0, p1, p2, fl, w, cx, cy, wn, rn, nb, gx, gy);
   }
   // outputs read only by later kernels: out_store, nontemporal on large
   // meshes, keeps L2 for the neighbour gathers (-1.5 % per step at 16M cells)
@@ -909,16 +974,20 @@ __global__ void k_reconstruct_one(DevMesh M, DevState S, DevWork W, int i, int k
   } else if (kind == 2) {
     double wn[3];
     NRec rn[3];
-    int jn[3];
+    bool pw[3], any_dry = false;
+#pragma unroll
     for (int kk = 0; kk < 3; ++kk) {
       int j = M.tt[kk * M.T + i];
       j = j < 0 ? i : j;  // a wall has no neighbour: the cell stands in, as in pass 1
-      jn[kk] = j;
       wn[kk] = S.w[S.at(j)];
       const CellRec r = M.crec[j];
       rn[kk] = NRec{r.cx, r.cy, (r.fl & CELL_BND) ? INFINITY : r.zmax, r.bc};
+      const bool full = rn[kk].zmx < wn[kk], wet = is_wet(wn[kk] - r.bc);
+      pw[kk] = !full && wet;
+      any_dry = any_dry || (!full && !wet);
+      if (pw[kk]) rn[kk].zmx = partwet1_w(r.zmin, r.zmin, r.zmax, r.bc, wn[kk]);
     }
-    fullwet_plane<HEAD_GRAD>(M, p0, p1, p2, fl, w, ri.cx, ri.cy, wn, rn, jn, gx, gy);
+    if (!any_dry) fullwet_plane<HEAD_GRAD>(p0, p1, p2, fl, w, ri.cx, ri.cy, wn, rn, pw, gx, gy);
   } else {
     partwet2_muscl<HEAD_PW2>(M, S, W, i, lvl1, o0, gx, gy);
   }
