@@ -315,29 +315,54 @@ __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W
 // ReconstructPartWetCell2 (src/MUSCLObject.cpp:114-191) for every partially
 // wet cell (src/SpaceDisc.cpp:47-51).  The node maximum m_max_wp at the
 // lowest vertex is max(z, AtPoint of each incident cell's pass-1 MUSCL).
-__device__ inline double node_max_pass1(const DevMesh& M, const DevWork& W, int n, const V3& P) {
+// L (1 or 4) adjacent lanes share the node: lane `sub` takes every L-th cell
+// around it, kN of them at a time, and the lanes' maxima are combined at the
+// end.  Every load of the kN is issued before the first is used; past the
+// end the last cell is read again, which leaves the maximum as it is.
+template <int L>
+__device__ inline double node_max_pass1(const DevMesh& M, const DevWork& W, int n, const V3& P, int sub) {
   double mx = P.z;
-  int b = M.n2c_off[n], e = M.n2c_off[n + 1];
-  for (int q = b; q < e; ++q) {
-    const int c = M.n2c[q];
-    const int k = W.cls[c];
-    // pass-1 reconstruction of c: partially wet cells hold their pass-1
-    // level in wrec1 (zero gradient) while pass 2 rewrites mw in place
-    double w0 = W.mw[c], gx = W.mgx[c], gy = W.mgy[c];
-    if (k == 1) { w0 = W.wrec1[c]; gx = 0.; gy = 0.; }
-    double dx = P.x - M.cx[c], dy = P.y - M.cy[c];
-    double a = w0 + (gx * dx + gy * dy);
-    if (!((a - P.z) >= 0)) a = P.z;
-    mx = dmax(mx, a);
+  const int b = M.n2c_off[n], e = M.n2c_off[n + 1];
+  constexpr int kN = L == 1 ? 6 : 2;
+  for (int q = b; q < e; q += kN * L) {
+    int c[kN], k[kN];
+    double w0[kN], gx[kN], gy[kN], w1[kN];
+    CXY o[kN];
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
+      const int x = q + r * L + sub;
+      c[r] = M.n2c[x < e ? x : e - 1];
+    }
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
+      k[r] = W.cls[c[r]];
+      w0[r] = W.mw[c[r]];
+      gx[r] = W.mgx[c[r]];
+      gy[r] = W.mgy[c[r]];
+      w1[r] = W.wrec1[c[r]];  // written for partially wet cells, used for them alone
+      o[r] = M.cxy[c[r]];
+    }
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
+      // pass-1 reconstruction: partially wet cells hold their pass-1 level in
+      // wrec1 (zero gradient) while pass 2 rewrites mw in place
+      if (k[r] == 1) { w0[r] = w1[r]; gx[r] = 0.; gy[r] = 0.; }
+      double dx = P.x - o[r].x, dy = P.y - o[r].y;
+      double a = w0[r] + (gx[r] * dx + gy[r] * dy);
+      if (!((a - P.z) >= 0)) a = P.z;
+      mx = dmax(mx, a);
+    }
   }
+  // every lane starts from P.z, so ties keep its zero's sign in any order
+  for (int off = 1; off < L; off <<= 1) mx = dmax(mx, __shfl_xor(mx, off, 64));
   return mx;
 }
 
 // the final MUSCL (w0, gx, gy) of a partially wet cell i; w1: its pass-1
 // (PartWet1) level, the result where pass 2 falls back to it
-template <bool HEAD_PW2>
-__device__ inline void partwet2_muscl(const DevMesh& M, const DevState& S, const DevWork& W, int i, double w1,
-                                      double& w0_out, double& gx_out, double& gy_out) {
+template <bool HEAD_PW2, int L>
+__device__ inline void partwet2_muscl(const DevMesh& M, const DevState& S, const DevWork& W, int i, int sub,
+                                      double w1, double& w0_out, double& gx_out, double& gy_out) {
   int i0 = M.tp[i], i1 = M.tp[M.T + i], i2 = M.tp[2 * M.T + i];
   V3 Q0 = node(M, i0), Q1 = node(M, i1), Q2 = node(M, i2);
   const double cx = M.cx[i], cy = M.cy[i], bc = M.bc[i];
@@ -355,7 +380,7 @@ __device__ inline void partwet2_muscl(const DevMesh& M, const DevState& S, const
   double w0 = w1, gx = 0., gy = 0.;  // fallback: pass-1 (PartWet1) result
   bool fallback = (w > b13) || (b13 - b23 < kTol);
   if (!fallback) {
-    double w23 = node_max_pass1(M, W, i0, Q0);
+    double w23 = node_max_pass1<L>(M, W, i0, Q0, sub);
     double h23 = w23 - b23;
     double ratio_b = (b12 - b23) / (b13 - b23);
     double hd1 = 1. / 3. * h23 * ratio_b;
@@ -401,22 +426,35 @@ __device__ inline void partwet2_muscl(const DevMesh& M, const DevState& S, const
   gy_out = gy;
 }
 
-template <bool HEAD_PW2>
-__device__ inline void recon2_cell(const DevMesh& M, const DevState& S, const DevWork& W, int i) {
+template <bool HEAD_PW2, int L>
+__device__ inline void recon2_cell(const DevMesh& M, const DevState& S, const DevWork& W, int i, int sub) {
   double w0, gx, gy;
-  partwet2_muscl<HEAD_PW2>(M, S, W, i, W.wrec1[i], w0, gx, gy);
+  partwet2_muscl<HEAD_PW2, L>(M, S, W, i, sub, W.wrec1[i], w0, gx, gy);
+  if (sub != 0) return;
   // in place: readers of pass-1 values take partially wet cells from wrec1
   W.mw[i] = w0;
   W.mgx[i] = gx;
   W.mgy[i] = gy;
 }
 
-// over the list of partially wet cells written by k_recon1
+// Over the list of partially wet cells written by k_recon1.  Short lists are
+// bound by one wave's gathers (~6 cells around a node, six arrays, a cache
+// line per lane each, through one CU's address unit): workgroups of one wave
+// spread them over the CUs, and while the launch has the lanes four of them
+// share a cell's gathers (they repeat its arithmetic, so longer lists take
+// a lane per cell).  Us per launch, 256-thread workgroups with a cell after
+// the other / now: 9.8 / 7.1 (Thacker bowl, 1,600 cells), 13.2 / 7.8
+// (40,000), dam break 20.4 / 8.3 (250k), 28.8 / 11.7 (4M).
+constexpr int kRecon2Block = 64;
 template <bool HEAD_PW2>
-__global__ void __launch_bounds__(256) k_recon2(DevMesh M, DevState S, DevWork W) {
-  const unsigned int n = *W.pw_count;
-  for (unsigned int q = blockIdx.x * kBlock + threadIdx.x; q < n; q += gridDim.x * kBlock)
-    recon2_cell<HEAD_PW2>(M, S, W, W.pw_list[q]);
+__global__ void __launch_bounds__(kRecon2Block) k_recon2(DevMesh M, DevState S, DevWork W) {
+  const unsigned int n = *W.pw_count, stride = gridDim.x * kRecon2Block;
+  const unsigned int t = blockIdx.x * kRecon2Block + threadIdx.x;
+  if (n <= stride / 4) {
+    if (t / 4 < n) recon2_cell<HEAD_PW2, 4>(M, S, W, W.pw_list[t / 4], (int)(t & 3));
+  } else {
+    for (unsigned int q = t; q < n; q += stride) recon2_cell<HEAD_PW2, 1>(M, S, W, W.pw_list[q], 0);
+  }
 }
 __global__ void k_zero_count(unsigned int* c) { *c = 0u; }
 
@@ -989,7 +1027,7 @@ __global__ void k_reconstruct_one(DevMesh M, DevState S, DevWork W, int i, int k
     }
     if (!any_dry) fullwet_plane<HEAD_GRAD>(p0, p1, p2, fl, w, ri.cx, ri.cy, wn, rn, pw, gx, gy);
   } else {
-    partwet2_muscl<HEAD_PW2>(M, S, W, i, lvl1, o0, gx, gy);
+    partwet2_muscl<HEAD_PW2, 1>(M, S, W, i, 0, lvl1, o0, gx, gy);
   }
   out[0] = o0; out[1] = o1; out[2] = o2; out[3] = gx; out[4] = gy;
 }
@@ -1073,10 +1111,10 @@ hipError_t launch_recon1(const DevMesh& M, const DevState& S, const DevWork& W, 
 }
 hipError_t launch_recon2(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
                          hipStream_t st) {
-  dim3 g = grid_for(M.c1 - M.c0);
+  dim3 g = grid_for_bs(4 * (M.c1 - M.c0), kRecon2Block);
   if (g.x > 1024) g.x = 1024;  // grid-stride over the list
-  if (opts & 2) hipLaunchKernelGGL((k_recon2<true>), g, dim3(256), 0, st, M, S, W);
-  else hipLaunchKernelGGL((k_recon2<false>), g, dim3(256), 0, st, M, S, W);
+  if (opts & 2) hipLaunchKernelGGL((k_recon2<true>), g, dim3(kRecon2Block), 0, st, M, S, W);
+  else hipLaunchKernelGGL((k_recon2<false>), g, dim3(kRecon2Block), 0, st, M, S, W);
   return hipGetLastError();
 }
 __global__ void __launch_bounds__(256) k_relayout(DevState S, DevOut O, int64_t T) {
