@@ -62,6 +62,8 @@ struct swe_solver {
   // after a fused stage W holds no fluxes: they are recomputed from the
   // stage's input buffer on demand (materialize_fluxes)
   bool flux_stale = false;
+  // W's pass-2 list is empty: the last stage cleared its length after use
+  bool pw_clean = false;
   int stale_in = -1, stale_slot = 0;
 };
 
@@ -135,6 +137,17 @@ int materialize_fluxes(swe_solver* s) {
   return SWE_OK;
 }
 
+// Both passes of the reconstruction of S into W; r: see launch_recon1.  W's
+// list is left in use: a stage whose last kernel clears it (pw_clear) sets
+// pw_clean again.
+hipError_t reconstruct(swe_solver* s, const DevState& S, unsigned long long* r = nullptr) {
+  const bool clean = s->pw_clean;
+  s->pw_clean = false;
+  hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, r);
+  if (e == hipSuccess) e = launch_recon2(s->M, S, s->W, s->opts, s->stream);
+  return e;
+}
+
 // a stage takes the fused kernel when its step size is known before the
 // flux pass: a fixed dt, or a later stage of a CFL step (slot > 0)
 bool use_fused(const swe_solver* s, double dt_fixed, int slot) {
@@ -149,17 +162,19 @@ bool use_fused_after_flux(const swe_solver* s) { return s->fused_ok && s->fused_
 int run_stage(swe_solver* s, int in, int u0, int out, double a0, double a1, double coef,
               double dt_fixed, double cfl, int slot, double* dts_log) {
   DevState S = state_of(s, in);
-  SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-  SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+  const bool fuse = use_fused(s, dt_fixed, slot);
+  SWE_CHECK(reconstruct(s, S, fuse ? nullptr : s->rbits + slot), "reconstruction");
   StageArgs A{a0, a1, coef, dt_fixed, cfl, s->cor, s->rbits, dts_log, friction(s)};
-  if (use_fused(s, dt_fixed, slot)) {
+  A.pw_clear = s->W.pw_count;
+  if (fuse) {
     SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, u0), out_of(s, out), s->W, A, s->flux, s->ws, s->opts,
                            s->stream), "fused");
     s->flux_stale = true;
     s->stale_in = in;
     s->stale_slot = slot;
   } else {
-    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + slot, s->flux_items, s->flux_block, s->stream), "flux");
+    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + slot, s->flux_items, s->flux_block, s->stream,
+                          kCflTake), "flux");
     s->flux_stale = false;
     if (use_fused_after_flux(s)) {
       SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, u0), out_of(s, out), s->W, A, s->flux, s->ws, s->opts,
@@ -169,6 +184,7 @@ int run_stage(swe_solver* s, int in, int u0, int out, double a0, double a1, doub
       SWE_CHECK(launch_update(s->M, S, state_of(s, u0), out_of(s, out), s->W, A, s->upd_items, s->upd_block, s->stream), "update");
     }
   }
+  s->pw_clean = true;
   s->last_r_slot = slot;
   return SWE_OK;
 }
@@ -350,10 +366,10 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
   for (int b = 0; b < 3; ++b) {
     if ((e = hipMemset(s->sbuf[b], 0, sizeof(double) * size_t(3 * s->Tpad))) != hipSuccess) return bail(e, "hipMemset");
   }
-  // the whole mesh is the visited window; cinst / bdt / bactive are set for
+  // the whole mesh is the visited window; cinst and the members' controls are set for
   // ensembles below
   s->M = DevMesh{dpx, dpy, dpz, dtp, dte, dtt, dfl, dep0, dep1, det0, det1, doff, dn2c, T, E, V,
-                 G.cx, G.cy, G.bc, G.area, G.edmin, G.crec, nullptr, nullptr, nullptr, 0, T, 0, E,
+                 G.cx, G.cy, G.bc, G.area, G.edmin, G.crec, nullptr, nullptr, nullptr, nullptr, 0, T, 0, E,
                  T >= (int64_t(1) << 20) ? 1 : 0, nullptr, (options & SWE_OPT_EXACT_BALANCE) ? 1 : 0, G.nrec, G.cxy, G.pn, G.cv};
   s->G = G;
   if (!pe.empty()) {
@@ -399,13 +415,14 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
     B.n = n_inst;
 #define ALLOC(ptr, n) if ((e = dalloc(s, &ptr, n)) != hipSuccess) return bail(e, "hipMalloc")
     ALLOC(dci, T);
-    ALLOC(B.t, n_inst); ALLOC(B.dt, n_inst); ALLOC(B.active, n_inst); ALLOC(B.steps, n_inst);
+    ALLOC(B.t, n_inst); ALLOC(B.active, n_inst); ALLOC(B.steps, n_inst);
     ALLOC(B.rbits, 4 * n_inst); ALLOC(B.n_active, 1);
 #undef ALLOC
     if ((e = hipMemcpy(dci, cell_inst->data(), sizeof(int) * size_t(T), hipMemcpyHostToDevice)) != hipSuccess)
       return bail(e, "hipMemcpy");
     s->M.cinst = dci;
-    s->M.bdt = B.dt;
+    s->M.br = B.rbits;
+    s->M.bt = B.t;
     s->M.bactive = B.active;
     if (int rc = swe_batch_reset(s, 0.0)) { swe_destroy(s); return rc; }
   }
@@ -516,8 +533,7 @@ int swe_compute_interface_values(swe_solver* s) {
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;
   DevState S = state_of(s, s->cur);
-  SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-  SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+  SWE_CHECK(reconstruct(s, S), "reconstruction");
   SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
   return SWE_OK;
 }
@@ -611,8 +627,7 @@ int swe_reconstruct(swe_solver* s, int64_t cell, int kind, double* out5) {
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;
   DevState S = state_of(s, s->cur);
-  SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-  SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+  SWE_CHECK(reconstruct(s, S), "reconstruction");
   double* d = nullptr;
   SWE_CHECK(hipMalloc((void**)&d, 5 * sizeof(double)), "hipMalloc");
   hipError_t e = launch_reconstruct_one(s->M, S, s->W, int(cell), kind, s->opts, d, s->stream);
@@ -750,18 +765,17 @@ static int batch_step(swe_solver* s, int scheme, double cfl, double t_end) {
   for (int q = 0; q < nst; ++q) {
     DevState S = state_of(s, st[q].in);
     StageArgs A{st[q].a0, st[q].a1, st[q].coef, 0., cfl, s->cor, nullptr, nullptr, friction(s)};
+    A.t_end = t_end;
+    A.pw_clear = s->W.pw_count;
+    SWE_CHECK(reconstruct(s, S), "reconstruction");
+    s->pw_clean = true;  // by this stage's last kernel
     if (q > 0 && use_fused(s, 0., q)) {  // the members' step sizes are known: one fused kernel
-      SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-      SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
       SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->flux, s->ws,
                              s->opts, s->stream), "fused");
       continue;
     }
-    SWE_CHECK(launch_batch_reset_r(s->B, q, s->stream), "batch_reset_r");
-    SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-    SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+    // slot 0 holds the step's r, set to 1 at the end of the step before
     SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->B.rbits + q, s->flux_items, s->flux_block, s->stream), "flux");
-    if (q == 0) SWE_CHECK(launch_batch_dt(s->B, cfl, t_end, s->stream), "batch_dt");
     if (use_fused_after_flux(s)) {
       SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->flux, s->ws,
                              s->opts, s->stream, false, true), "fused from fluxes");
@@ -771,7 +785,7 @@ static int batch_step(swe_solver* s, int scheme, double cfl, double t_end) {
     SWE_CHECK(launch_update(s->M, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->upd_items, s->upd_block, s->stream),
               "update");
   }
-  SWE_CHECK(launch_batch_advance(s->B, t_end, s->stream), "batch_advance");
+  SWE_CHECK(launch_batch_advance(s->B, cfl, t_end, s->stream), "batch_advance");
   if (scheme == SWE_SCHEME_EULER) s->cur = b;
   return SWE_OK;
 }
@@ -780,11 +794,10 @@ int swe_batch_reset(swe_solver* s, double t0) {
   if (!s || s->n_inst <= 0) return fail(SWE_ERR_ARG, "not an ensemble solver");
   if (int rc = set_device(s)) return rc;
   const int n = s->n_inst;
-  std::vector<double> t(size_t(n), t0), dt(size_t(n), 0.);
+  std::vector<double> t(size_t(n), t0);
   std::vector<int> act(size_t(n), 1);
   std::vector<long long> steps(size_t(n), 0);
   SWE_CHECK(hipMemcpy(s->B.t, t.data(), sizeof(double) * size_t(n), hipMemcpyHostToDevice), "hipMemcpy");
-  SWE_CHECK(hipMemcpy(s->B.dt, dt.data(), sizeof(double) * size_t(n), hipMemcpyHostToDevice), "hipMemcpy");
   SWE_CHECK(hipMemcpy(s->B.active, act.data(), sizeof(int) * size_t(n), hipMemcpyHostToDevice), "hipMemcpy");
   SWE_CHECK(hipMemcpy(s->B.steps, steps.data(), sizeof(long long) * size_t(n), hipMemcpyHostToDevice), "hipMemcpy");
   SWE_CHECK(hipMemcpy(s->B.n_active, &n, sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
@@ -836,9 +849,18 @@ static int batch_window(swe_solver* s, const std::vector<int>& act, bool euler) 
   return copy(std::max(oc0, s->M.c1), oc1);
 }
 
+// empties W's pass-2 list where the last user left it in use
+static int clean_list(swe_solver* s) {
+  if (s->pw_clean) return SWE_OK;
+  SWE_CHECK(launch_zero_count(s->W.pw_count, s->stream), "zero_count");
+  s->pw_clean = true;
+  return SWE_OK;
+}
+
 static int batch_capture(swe_solver* s, int scheme, double cfl, double t_end, int per_graph) {
   if (s->graph) { (void)hipGraphExecDestroy(s->graph); s->graph = nullptr; }
   const int cur0 = s->cur;
+  if (int rc = clean_list(s)) return rc;  // the captured steps start and end with W's list empty
   hipGraph_t g;
   SWE_CHECK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
   int rc = SWE_OK;
@@ -873,6 +895,8 @@ int swe_batch_run(swe_solver* s, int scheme, double cfl, double t_end, int64_t m
   SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
   const bool euler = scheme == SWE_SCHEME_EULER;
   if (int rc = batch_window(s, act_flags, euler)) return rc;
+  if (int rc = clean_list(s)) return rc;
+  SWE_CHECK(launch_batch_reset_r(s->B, 0, s->stream), "batch_reset_r");
   int64_t done = 0;
   int act = 0;
   for (int f : act_flags) act += f;
@@ -1001,9 +1025,14 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
           if (e == hipSuccess) e = hipEventRecord(ev[size_t(2 * q + 1)], s->stream);
           used[q] = true;
         };
-        timed(0, [&] { return launch_recon1(s->M, S, s->W, s->opts, s->stream); });
+        A.pw_clear = s->W.pw_count;
+        const bool clean = s->pw_clean, fuse = use_fused(s, dt, st);
+        s->pw_clean = false;
+        timed(0, [&] {
+          return launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, fuse ? nullptr : s->rbits + st);
+        });
         timed(1, [&] { return launch_recon2(s->M, S, s->W, s->opts, s->stream); });
-        if (use_fused(s, dt, st)) {
+        if (fuse) {
           timed(5, [&] {
             return launch_fused(s->M, s->tiles, S, state_of(s, u0), out_of(s, out), s->W, A, s->flux, s->ws,
                                 s->opts, s->stream);
@@ -1014,7 +1043,7 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
         } else {
           timed(2, [&] {
             return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + st, s->flux_items, s->flux_block,
-                               s->stream);
+                               s->stream, kCflTake);
           });
           s->flux_stale = false;
           if (use_fused_after_flux(s)) {
@@ -1032,6 +1061,7 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
         }
         if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) { rc = dev_fail(e, "kernel"); break; }
+        s->pw_clean = true;
         for (int q = 0; q < nk; ++q) {
           if (!used[q]) continue;
           float f = 0.f;
@@ -1126,8 +1156,7 @@ int swe_autotune(swe_solver* s, int reps, int* flux_items, int* update_items, do
   DevState S = state_of(s, s->cur);
   const int scratch = (s->cur + 1) % 3;
   unsigned long long* rslot = (s->n_inst > 0 ? s->B.rbits : s->rbits) + 3;
-  SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-  SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+  SWE_CHECK(reconstruct(s, S), "reconstruction");
   hipEvent_t e0, e1;
   SWE_CHECK(hipEventCreate(&e0), "hipEventCreate");
   SWE_CHECK(hipEventCreate(&e1), "hipEventCreate");
@@ -1299,8 +1328,7 @@ int swe_integrals(swe_solver* s, double* out3, double* per_cell) {
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;
   DevState S = state_of(s, s->cur);
-  SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-  SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+  SWE_CHECK(reconstruct(s, S), "reconstruction");
   const int64_t nb = integrals_blocks(s->M);
   double *d = nullptr, *pc = nullptr;
   SWE_CHECK(hipMalloc((void**)&d, sizeof(double) * size_t(3 * nb + 3)), "hipMalloc");
@@ -1332,8 +1360,7 @@ int swe_integrals_noalloc(swe_solver* s, double* out3_dev, double* per_cell_dev)
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;
   DevState S = state_of(s, s->cur);
-  SWE_CHECK(launch_recon1(s->M, S, s->W, s->opts, s->stream), "recon1");
-  SWE_CHECK(launch_recon2(s->M, S, s->W, s->opts, s->stream), "recon2");
+  SWE_CHECK(reconstruct(s, S), "reconstruction");
   SWE_CHECK(launch_integrals(s->M, S, s->W, s->scratch, per_cell_dev, out3_dev, s->stream), "integrals");
   return SWE_OK;
 }
@@ -1603,7 +1630,7 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
         } else {
           if (e == hipSuccess)  // fixed dt: the CFL reduction is not read
             e = launch_flux(s->M, Sq, Wq, s->flux, s->ws, s->cor, s->rbits + 3, s->flux_items, s->flux_block, s->stream,
-                            false);
+                            kCflOff);
           if (use_fused_after_flux(s)) {  // draining (stored) and update in one tile kernel
             if (e == hipSuccess)
               e = launch_fused(s->M, s->tiles, Sq, Un, O, Wq, A, s->flux, s->ws, s->opts, s->stream, true, true);

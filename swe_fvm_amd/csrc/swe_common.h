@@ -177,6 +177,24 @@ __device__ __forceinline__ void rhs_compute(const RhsIn& q, double dts, double c
       },
       dts, cor, fric, eb, r0, r1, r2);
 }
+// the stage's step size: fixed, or cfl times r of the step's first flux pass
+__device__ __forceinline__ double stage_dt(const StageArgs& A) {
+  double dt = A.dt_fixed;
+  if (!(dt > 0.)) dt = A.cfl * __longlong_as_double((long long)A.rbits[0]);
+  return dt;
+}
+// an ensemble member's: cfl * r, clipped so that the last step lands on
+// t_end (every stage and the end of the step compute it from the same r and
+// t, which nothing changes in between)
+__device__ __forceinline__ double batch_dt(unsigned long long r, double t, double cfl, double t_end) {
+  double d = cfl * __longlong_as_double((long long)r);
+  const double rest = t_end - t;
+  if (!(d < rest)) d = rest;
+  return d;
+}
+__device__ __forceinline__ double member_dt(const DevMesh& M, const StageArgs& A, int inst) {
+  return batch_dt(M.br[4 * (int64_t)inst], M.bt[inst], A.cfl, A.t_end);
+}
 // grid of 256-thread workgroups covering n items, a multiple of 8 (one
 // contiguous range per XCD, see logical_block)
 // a store of a kernel output; NT (a template parameter: a runtime branch

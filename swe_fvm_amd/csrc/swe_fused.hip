@@ -33,12 +33,6 @@
 
 namespace swe {
 
-__device__ __forceinline__ double stage_dt_fused(const StageArgs& A) {
-  double dt = A.dt_fixed;
-  if (!(dt > 0.)) dt = A.cfl * __longlong_as_double((long long)A.rbits[0]);
-  return dt;
-}
-
 // waves per SIMD the register allocation must allow, and threads per tile
 // workgroup (kTileCells or 2 kTileCells: the flux and draining phases then
 // give each thread fewer items, the update leaves the second half idle);
@@ -61,6 +55,7 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
   // the evaluating instance walks the tiles backwards (it follows a
   // forward reconstruction); the FF instance forwards (it follows k_flux)
   const int64_t tile = t0 + (FF ? logical_block() : logical_block_reversed());
+  if (A.pw_clear && blockIdx.x == 0 && threadIdx.x == 0) *A.pw_clear = 0u;
   if (tile >= t1) return;  // padding workgroups of the XCD-aware grid
   const int64_t c0 = tile * kTileCells;
   const int nc = (int)(M.T - c0 < kTileCells ? M.T - c0 : kTileCells);
@@ -240,7 +235,7 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
   // ---- update of the tile's cells (k_update's operations; the fluxes and
   // neighbour draining steps are read from LDS edge by edge)
   if (!mine) return;
-  const double dt = M.cinst ? 0. : stage_dt_fused(A);
+  const double dt = M.cinst ? 0. : stage_dt(A);
   if (A.dts_log && tile == 0 && tid == 0) A.dts_log[0] = dt;
   double dts = A.coef * dt;
   if (M.cinst) {  // ensembles: the member's own step size (k_update's rule)
@@ -254,7 +249,7 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
       O.v[o] = comb ? v0 : v;
       return;
     }
-    dts = A.coef * M.bdt[inst];
+    dts = A.coef * member_dt(M, A, inst);
   }
   q.dti = sD[tid];
   const double bc = centroid(q.p[0], q.p[1], q.p[2]).z;

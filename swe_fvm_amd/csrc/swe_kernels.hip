@@ -154,7 +154,7 @@ __device__ __forceinline__ void fullwet_plane(const V3& p0, const V3& p1, const 
 // 28.7 / 13.5 (250k cells), 40 / 27.9 (1M), 100 / 92.5 (4M); without
 // partially wet cells 4.9 / 4.9 (62k).
 template <bool HEAD_GRAD, bool NT>
-__global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W) {
+__global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W, unsigned long long* r) {
   // The workgroup's 256 Morton-consecutive cells stage their level and the
   // part of their record a neighbour reads (NRec) in LDS; most neighbours
   // lie in the same workgroup and are read from there, the others from
@@ -208,6 +208,7 @@ __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W
     sh.win.r[tid] = ri;
   }
   if (tid == 0) s_n = 0;
+  if (r && blockIdx.x == 0 && tid == 0) *r = (unsigned long long)__double_as_longlong(1.0);
   __syncthreads();
   // finished ensemble members are left alone
   const bool on = live && !(M.cinst && !M.bactive[M.cinst[is]]);
@@ -662,12 +663,6 @@ __device__ __forceinline__ void rhs_cell(const DevMesh& M, const DevState& S, co
   rhs_compute(q, dts, cor, fric, M.eb != 0, r0, r1, r2);
 }
 
-__device__ __forceinline__ double stage_dt(const StageArgs& A) {
-  double dt = A.dt_fixed;
-  if (!(dt > 0.)) dt = A.cfl * __longlong_as_double((long long)A.rbits[0]);
-  return dt;
-}
-
 // NI cells per thread, BS apart (BS threads per workgroup), loads of all of
 // them first (NI and BS are launch-time choices like the flux's).
 template <int NI, int BS, bool NT>
@@ -676,6 +671,7 @@ __global__ void __launch_bounds__(BS) k_update(DevMesh M, DevState S, DevState U
   const int64_t base = M.c0 + (int64_t)logical_block() * (BS * NI) + threadIdx.x;
   const double dt = M.cinst ? 0. : stage_dt(A);
   if (A.dts_log && blockIdx.x == 0 && threadIdx.x == 0) A.dts_log[0] = dt;
+  if (A.pw_clear && blockIdx.x == 0 && threadIdx.x == 0) *A.pw_clear = 0u;
   RhsIn in[NI];
   double w[NI], u[NI], v[NI], bc[NI];
   double w0[NI], u0[NI], v0[NI];
@@ -709,7 +705,7 @@ __global__ void __launch_bounds__(BS) k_update(DevMesh M, DevState S, DevState U
         O.v[O.at(i)] = comb ? v0[it] : v[it];
         continue;
       }
-      dts = A.coef * M.bdt[inst];
+      dts = A.coef * member_dt(M, A, inst);
     }
     double R0, R1, R2;
     rhs_compute(in[it], dts, A.cor, A.fric, M.eb != 0, R0, R1, R2);
@@ -746,32 +742,19 @@ __global__ void k_batch_reset_r(DevBatch B, int slot) {
   if (k < B.n) B.rbits[4 * k + slot] = (unsigned long long)__double_as_longlong(1.0);
 }
 
-// dt of every active member after the step's first flux pass: cfl * r,
-// clipped so the last step lands on t_end.
-__global__ void k_batch_dt(DevBatch B, double cfl, double t_end) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= B.n) return;
-  double d = 0.;
-  if (B.active[k]) {
-    d = cfl * __longlong_as_double((long long)B.rbits[4 * k]);
-    double rest = t_end - B.t[k];
-    if (!(d < rest)) d = rest;
-  }
-  B.dt[k] = d;
-}
-
 // end of a step: advance time, retire members that reached t_end, count
-// the active ones (one workgroup of 1024 threads, strided over members)
-__global__ void __launch_bounds__(1024) k_batch_advance(DevBatch B, double t_end) {
+// the active ones, and reset r for the next step's first flux pass (one
+// workgroup of 1024 threads, strided over members)
+__global__ void __launch_bounds__(1024) k_batch_advance(DevBatch B, double cfl, double t_end) {
   __shared__ int cnt;
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
   int mine = 0;
   for (int k = threadIdx.x; k < B.n; k += blockDim.x) {
     if (B.active[k]) {
-      double d = B.dt[k];
-      double t = B.t[k];
-      double rest = t_end - t;
+      const double t = B.t[k], rest = t_end - t;
+      const double d = batch_dt(B.rbits[4 * k], t, cfl, t_end);
+      B.rbits[4 * k] = (unsigned long long)__double_as_longlong(1.0);
       B.t[k] = (d < rest) ? t + d : t_end;
       B.steps[k] += 1;
       B.active[k] = (d < rest) ? 1 : 0;
@@ -1097,16 +1080,20 @@ hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStrea
   return hipGetLastError();
 }
 hipError_t launch_recon1(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
-                         hipStream_t st, bool zero_count) {
+                         hipStream_t st, bool zero_count, unsigned long long* r) {
   if (zero_count) hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, st, W.pw_count);
   const dim3 g = grid_for(M.c1 - M.c0);
   if (opts & 1) {
-    if (M.nt) hipLaunchKernelGGL((k_recon1<true, true>), g, dim3(256), 0, st, M, S, W);
-    else hipLaunchKernelGGL((k_recon1<true, false>), g, dim3(256), 0, st, M, S, W);
+    if (M.nt) hipLaunchKernelGGL((k_recon1<true, true>), g, dim3(256), 0, st, M, S, W, r);
+    else hipLaunchKernelGGL((k_recon1<true, false>), g, dim3(256), 0, st, M, S, W, r);
   } else {
-    if (M.nt) hipLaunchKernelGGL((k_recon1<false, true>), g, dim3(256), 0, st, M, S, W);
-    else hipLaunchKernelGGL((k_recon1<false, false>), g, dim3(256), 0, st, M, S, W);
+    if (M.nt) hipLaunchKernelGGL((k_recon1<false, true>), g, dim3(256), 0, st, M, S, W, r);
+    else hipLaunchKernelGGL((k_recon1<false, false>), g, dim3(256), 0, st, M, S, W, r);
   }
+  return hipGetLastError();
+}
+hipError_t launch_zero_count(unsigned int* count, hipStream_t st) {
+  hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, st, count);
   return hipGetLastError();
 }
 hipError_t launch_recon2(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
@@ -1131,11 +1118,9 @@ hipError_t launch_relayout(const DevState& S, const DevOut& O, int64_t T, hipStr
 }
 hipError_t launch_flux(const DevMesh& M, const DevState& S, const DevWork& W, int flux, int ws,
                        double cor, unsigned long long* rbits, int items, int block, hipStream_t st,
-                       bool reset) {
-  // without the reset (a fixed-dt pass of a single mesh) the minimum is not
-  // taken at all; ensembles always take their per-member minima
-  const bool cfl = reset || M.cinst;
-  if (reset && !M.cinst) hipLaunchKernelGGL(k_reset_r, dim3(1), dim3(1), 0, st, rbits);
+                       CflMode mode) {
+  const bool cfl = mode != kCflOff || M.cinst;  // ensembles always take their members' minima
+  if (mode == kCflReset && !M.cinst) hipLaunchKernelGGL(k_reset_r, dim3(1), dim3(1), 0, st, rbits);
   if (M.e1 <= M.e0) return hipGetLastError();
   if (block != 256 && block != 512) return hipErrorInvalidValue;
   dim3 g = grid_for_bs((M.e1 - M.e0 + items - 1) / items, block), b(block);
@@ -1187,12 +1172,8 @@ hipError_t launch_batch_reset_r(const DevBatch& B, int slot, hipStream_t st) {
   hipLaunchKernelGGL(k_batch_reset_r, dim3((B.n + 255) / 256), dim3(256), 0, st, B, slot);
   return hipGetLastError();
 }
-hipError_t launch_batch_dt(const DevBatch& B, double cfl, double t_end, hipStream_t st) {
-  hipLaunchKernelGGL(k_batch_dt, dim3((B.n + 255) / 256), dim3(256), 0, st, B, cfl, t_end);
-  return hipGetLastError();
-}
-hipError_t launch_batch_advance(const DevBatch& B, double t_end, hipStream_t st) {
-  hipLaunchKernelGGL(k_batch_advance, dim3(1), dim3(1024), 0, st, B, t_end);
+hipError_t launch_batch_advance(const DevBatch& B, double cfl, double t_end, hipStream_t st) {
+  hipLaunchKernelGGL(k_batch_advance, dim3(1), dim3(1024), 0, st, B, cfl, t_end);
   return hipGetLastError();
 }
 hipError_t launch_edge_field(const DevMesh& M, const DevState& S, const DevWork& W, double cor,

@@ -86,9 +86,10 @@ struct DevMesh {
   const double* edmin;
   const CellRec* crec;
   // batched ensembles (null for a single mesh): instance of every cell and
-  // the per-instance step size and activity flag
+  // the per-instance r (4 slots apart), simulated time and activity flag
   const int* cinst;
-  const double* bdt;
+  const unsigned long long* br;
+  const double* bt;
   const int* bactive;
   // cells [c0, c1) and edges [e0, e1) the step kernels visit (the whole mesh
   // except when finished ensemble members are trimmed off the front)
@@ -119,7 +120,6 @@ struct DevMesh {
 struct DevBatch {
   int n;                      // instances
   double* t;                  // simulated time
-  double* dt;                 // step size of the current step
   int* active;                // t < t_end
   long long* steps;           // steps taken
   unsigned long long* rbits;  // r of each flux pass, 4 slots per instance
@@ -231,32 +231,41 @@ struct StageArgs {
   const unsigned long long* rbits;  // r of the step's first flux pass (double bits)
   double* dts_log;     // receives the step's dt (first stage only), may be null
   double fric;         // linear friction coefficient (0: none)
+  double t_end = 0.;   // ensembles: the members' last time
+  // zeroed by the stage's last kernel (pass 2 has read it), for the next
+  // stage's reconstruction; null where the count is kept
+  unsigned int* pw_clear = nullptr;
 };
 
 // the state of cells [0, T) rewritten from S's layout into O's
 hipError_t launch_relayout(const DevState& S, const DevOut& O, int64_t T, hipStream_t st);
 hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStream_t st);
-// zero_count false: the caller has zeroed W.pw_count (launch_slot_counts)
+// zero_count false: W.pw_count is zero already (the stage before cleared it,
+// or launch_slot_counts); r (may be null): set to 1, for the flux pass that
+// follows
 hipError_t launch_recon1(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
-                         hipStream_t st, bool zero_count = true);
+                         hipStream_t st, bool zero_count = true, unsigned long long* r = nullptr);
+hipError_t launch_zero_count(unsigned int* count, hipStream_t st);
 hipError_t launch_recon2(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
                          hipStream_t st);
 // items: edges per thread of the flux (1, 2 or 4), cells per thread of the
 // update (1 or 2); block: threads per workgroup of either (256 or 512);
 // results are identical for every choice
-// reset false (single mesh): no CFL minimum at all, neither reset nor taken
-// (a fixed-dt pass that never reads it); the fluxes are the same
+// kCflOff (single mesh): no CFL minimum (a fixed-dt pass that never reads
+// it); kCflTake: the minimum into r, which the reconstruction before has set
+// to 1; kCflReset: the same with a launch of its own that sets it.  The
+// fluxes are the same.
+enum CflMode { kCflOff, kCflTake, kCflReset };
 hipError_t launch_flux(const DevMesh& M, const DevState& S, const DevWork& W, int flux, int ws,
                        double cor, unsigned long long* rbits, int items, int block, hipStream_t st,
-                       bool reset = true);
+                       CflMode cfl = kCflReset);
 // opts & 32 (SWE_OPT_DRAIN_LENGTH): outflow F0 * L in the draining dt
 hipError_t launch_drain(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
                         hipStream_t st);
 hipError_t launch_update(const DevMesh& M, const DevState& S, const DevState& U0, const DevOut& O,
                          const DevWork& W, const StageArgs& A, int items, int block, hipStream_t st);
 hipError_t launch_batch_reset_r(const DevBatch& B, int slot, hipStream_t st);
-hipError_t launch_batch_dt(const DevBatch& B, double cfl, double t_end, hipStream_t st);
-hipError_t launch_batch_advance(const DevBatch& B, double t_end, hipStream_t st);
+hipError_t launch_batch_advance(const DevBatch& B, double cfl, double t_end, hipStream_t st);
 hipError_t launch_edge_field(const DevMesh& M, const DevState& S, const DevWork& W, double cor,
                              double* edg, double* src, hipStream_t st);
 hipError_t launch_max_wp(const DevMesh& M, const DevWork& W, double* out, hipStream_t st);

@@ -7,6 +7,8 @@ import pytest
 
 import swe_fvm_amd as swe
 from oracle import oracle as O
+from swe_fvm_amd import _lib
+from swe_fvm_amd.ensemble import Ensemble
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +60,38 @@ def test_partially_wet_lists_match_the_oracle(mesh, wet_share, opts):
         sd.run("SSPRK2", steps, dt=0.0, cfl=0.15)
         orc.run("SSPRK2", steps, dt=0.0, cfl=0.15)
         assert np.array_equal(sd.GetVolField(), orc.state())
+
+
+def test_list_reuse_across_getters_and_steps():
+    """Steps leave the list empty for the next reconstruction, the getters in use; any order of the two agrees."""
+    xyz, topo = swe.jittered_mesh(16, 0.3, 4)
+    prim = film(xyz, topo, 11, 0.3)
+    fl = swe.Fluxes.HLL[swe.Wavespeeds.Davis]
+    sd = swe.SpaceDisc(fl, swe.Domain(xyz, topo), prim)
+    orc = O.OracleSolver(xyz, topo.tables(), "HLL", "Davis")
+    orc.set_state(prim)
+    for scheme, fused, dt in (("SSPRK3", True, 0.0), ("Euler", True, 1e-4), ("SSPRK2", False, 0.0), ("SSPRK2", True, 0.0)):
+        sd.set_fused(fused)
+        sd.Integrals()
+        sd.run(scheme, 1, dt=dt)
+        sd.ComputeInterfaceValues()
+        sd.run(scheme, 2, dt=dt)
+        orc.run(scheme, 3, dt=dt, cfl=0.15)
+        assert np.array_equal(sd.GetVolField(), orc.state()), (scheme, fused)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_ensemble_steps_interrupted_by_a_reconstruction(graph):
+    members = [swe.jittered_mesh(n, 0.3, n) for n in (5, 16, 23)]
+    states = [film(x, t, k, 0.5) for k, (x, t) in enumerate(members)]
+    doms = [swe.Domain(x, t) for x, t in members]
+    fl = swe.Fluxes.HLLC[swe.Wavespeeds.Einfeldt]
+    out = []
+    for interrupt in (False, True):
+        ens = Ensemble(fl, doms, states)
+        for _ in range(3):
+            ens.run("SSPRK2", cfl=0.15, t_end=1.0, max_steps=4, graph=graph)
+            if interrupt:
+                assert _lib.load().swe_compute_interface_values(ens._h) == 0
+        out.append(np.concatenate(ens.states() + [ens.times()[0][:, None].repeat(3, 1)]))
+    assert np.array_equal(out[0], out[1])
