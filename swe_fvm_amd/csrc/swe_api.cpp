@@ -383,30 +383,34 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
   // the separate flux, draining and update kernels (ensembles tile their
   // stacked mesh; no edge joins two members)
   if (pe.empty()) {
-    TileTables tt_host;
-    if (build_tiles(T, tt.data(), te.data(), flag.data(), et0.data(), et1.data(), ep0.data(), ep1.data(), tt_host)) {
-      uint32_t *dcode, *drcode;
-      int *droff, *drcell, *devoff;
-      EdgeRec* dev;
-      int* devedge;
-#define ALLOC(ptr, n) if ((e = dalloc(s, &ptr, n)) != hipSuccess) return bail(e, "hipMalloc")
-#define H2D(dst, v)                                                                                      \
+    StageTables stt;
+    if (plain_geometry(V, px.data(), py.data(), E, ep0.data(), ep1.data()) &&
+        build_stage_tables(T, tp.data(), tt.data(), te.data(), flag.data(), et0.data(), et1.data(), ep0.data(),
+                           ep1.data(), stt)) {
+      TileHead* dhead;
+      TileCell* dcell;
+      int *dxcell, *dnode, *devedge;
+      RingCode* dxcode;
+      EvalCode* dev;
+      double *dtnode, *dtxc, *dtring;
+      const int64_t nt = stt.ntiles;
+#define UP(dst, v)                                                                                       \
+  if ((e = dalloc(s, &dst, int64_t(v.size()))) != hipSuccess) return bail(e, "hipMalloc");                \
   if (!v.empty() && (e = hipMemcpy(dst, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice)) != hipSuccess) \
     return bail(e, "hipMemcpy");
-      ALLOC(dcode, int64_t(tt_host.code.size())); ALLOC(droff, int64_t(tt_host.ring_off.size()));
-      ALLOC(drcell, int64_t(tt_host.ring_cell.size())); ALLOC(drcode, int64_t(tt_host.ring_code.size()));
-      ALLOC(devoff, int64_t(tt_host.ev_off.size())); ALLOC(dev, int64_t(tt_host.evrec.size()));
-      ALLOC(devedge, int64_t(tt_host.evedge.size()));
-      H2D(dcode, tt_host.code); H2D(droff, tt_host.ring_off); H2D(drcell, tt_host.ring_cell);
-      H2D(drcode, tt_host.ring_code); H2D(devoff, tt_host.ev_off); H2D(dev, tt_host.evrec);
-      H2D(devedge, tt_host.evedge);
-#undef H2D
+      UP(dhead, stt.head) UP(dcell, stt.cell) UP(dxcell, stt.xcell) UP(dxcode, stt.xcode) UP(dnode, stt.node)
+      UP(dev, stt.ev) UP(devedge, stt.evedge)
+#undef UP
+#define ALLOC(ptr, n) if ((e = dalloc(s, &ptr, n)) != hipSuccess) return bail(e, "hipMalloc")
+      ALLOC(dtnode, 3 * nt * stt.sn); ALLOC(dtxc, 2 * nt * stt.sx); ALLOC(dtring, 2 * nt * stt.sr);
 #undef ALLOC
-      s->tiles = DevTiles{dcode, droff, drcell, drcode, devoff, dev, devedge, tt_host.ntiles};
-      s->fused_ok = true;
+      s->tiles = DevTiles{dhead, dcell, dxcell, dxcode, dnode, dev, devedge, dtnode, dtxc, dtring, nt,
+                          stt.sx, stt.sr, stt.sn, stt.se, stt.max_own_nodes, stt.max_own_ev};
+      s->fused_ok = fused_fits(s->tiles);
     }
   }
   if ((e = launch_setup_geometry(s->M, G, s->stream)) != hipSuccess) return bail(e, "setup_geometry");
+  if (s->fused_ok && (e = launch_setup_tiles(s->M, s->tiles, s->stream)) != hipSuccess) return bail(e, "setup_tiles");
   if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) return bail(e, "hipStreamSynchronize");
   if (n_inst > 0) {
     s->n_inst = n_inst;
@@ -1803,6 +1807,7 @@ int swe_set_bathymetry(swe_solver* s, const double* z) {
     s->graph_scheme = -1;
   }
   SWE_CHECK(launch_setup_geometry(s->M, s->G, s->stream), "setup_geometry");
+  if (s->fused_ok) SWE_CHECK(launch_setup_tiles(s->M, s->tiles, s->stream), "setup_tiles");
   SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
   return SWE_OK;
 }

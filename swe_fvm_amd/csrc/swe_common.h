@@ -88,7 +88,8 @@ __device__ __forceinline__ Slot slot_value(const Muscl& m, double cx, double cy,
 // MUSCL, vertices and draining time step (RhsCell), and per local edge k
 // the edge's flux and the neighbour's draining time step, which the
 // accessor edge(k, F0, F1, F2, dtik) supplies (from registers in the
-// update kernel, from LDS in the fused kernel: the same arithmetic).
+// update kernel, from LDS in the fused kernel: the same arithmetic), and the
+// edge's nodes, which ends(k, Pa, Pb) supplies.
 struct RhsCell {
   uint32_t fl;
   Muscl mu;
@@ -102,8 +103,8 @@ struct RhsIn : RhsCell {
 // eb (SWE_OPT_EXACT_BALANCE): each edge adds the flux minus the cell's own
 // hydrostatic edge pressure, sg F - n h_ek^2 / 2, which is zero to the bit
 // where the edge states on both sides are equal and at rest
-template <class EdgeIn>
-__device__ __forceinline__ void rhs_compute_by(const RhsCell& q, EdgeIn edge, double dts, double cor,
+template <class Geometry, class EdgeIn, class Ends>
+__device__ __forceinline__ void rhs_compute_by(const RhsCell& q, EdgeIn edge, Ends ends, double dts, double cor,
                                                double fric, bool eb, double& r0, double& r1, double& r2) {
   r0 = 0.; r1 = 0.; r2 = 0.;
   // Domain::T / Area (src/Bathymetry.cpp:24-27,84-90)
@@ -118,9 +119,10 @@ __device__ __forceinline__ void rhs_compute_by(const RhsCell& q, EdgeIn edge, do
     const double dtk = (sg * F0) > 0. ? dmin(dts, q.dti) : dmin(dts, dtik);
     // Domain::L / E / Tang of edge k (src/Bathymetry.cpp:29-76); the tangent
     // is taken outward of this cell, as Norm(e, i) is
-    const V3 Pa = pick(q.p[0], q.p[1], q.p[2], ep0_local(q.fl, k));
-    const V3 Pb = pick(q.p[0], q.p[1], q.p[2], ep1_local(q.fl, k));
-    const double le = edge_len(Pa, Pb);
+    V3 Pa, Pb;
+    ends(k, Pa, Pb);
+    double le, tx, ty;
+    Geometry::edge(Pa, Pb, c, le, tx, ty);
     const double c_ek = i_area * le;
     const V3 E = midpoint(Pa, Pb);
     const Slot s = slot_value(q.mu, c.x, c.y, E);
@@ -128,8 +130,6 @@ __device__ __forceinline__ void rhs_compute_by(const RhsCell& q, EdgeIn edge, do
     double src1 = q.mu.gx, src2 = q.mu.gy;
     src1 += cor * (-s.v);
     src2 += cor * s.u;
-    double tx, ty;
-    tangent(Pa, Pb, le, c, tx, ty);
     const double nx = ty, ny = -tx;
     if (eb) {
       const double q2 = 0.5 * h_ek * h_ek;
@@ -170,10 +170,14 @@ __device__ __forceinline__ double stage_combine(bool cvx, double a0, double a1, 
 }
 __device__ __forceinline__ void rhs_compute(const RhsIn& q, double dts, double cor, double fric, bool eb,
                                             double& r0, double& r1, double& r2) {
-  rhs_compute_by(
+  rhs_compute_by<AnyGeometry>(
       q,
       [&](int k, double& F0, double& F1, double& F2, double& dtik) {
         F0 = q.F0[k]; F1 = q.F1[k]; F2 = q.F2[k]; dtik = q.dtik[k];
+      },
+      [&](int k, V3& Pa, V3& Pb) {
+        Pa = pick(q.p[0], q.p[1], q.p[2], ep0_local(q.fl, k));
+        Pb = pick(q.p[0], q.p[1], q.p[2], ep1_local(q.fl, k));
       },
       dts, cor, fric, eb, r0, r1, r2);
 }

@@ -33,104 +33,103 @@
 
 namespace swe {
 
-// waves per SIMD the register allocation must allow, and threads per tile
-// workgroup (kTileCells or 2 kTileCells: the flux and draining phases then
-// give each thread fewer items, the update leaves the second half idle);
-// build-time knobs
+// waves per SIMD the register allocation must allow; a build-time knob
 #ifndef SWE_FUSED_MIN_WAVES
 #define SWE_FUSED_MIN_WAVES 4
 #endif
-#ifndef SWE_FUSED_THREADS
-#define SWE_FUSED_THREADS 256
-#endif
-constexpr int kFusedThreads = SWE_FUSED_THREADS;
-static_assert(kFusedThreads == kTileCells || kFusedThreads == 2 * kTileCells, "threads per tile");
+// LDS of a tile, in doubles, the arrays one after the other: the
+// reconstruction of the local cells (w0, gx, gy, u, v, centroid) where the
+// fluxes are evaluated, the nodes (x, y, z), the fluxes.  The draining steps
+// take the place of the cells' w0, which nothing reads after the fluxes.
+__host__ __device__ __forceinline__ int lds_doubles(const DevTiles& P, bool ff, bool len) {
+  return (ff ? kTileCells + P.sr : 7 * (kTileCells + P.sx)) + 3 * (ff && !len ? P.lo : P.sn) + P.se + 2 * P.la;
+}
 
+__device__ __forceinline__ int local3(uint32_t word, int k) { return (int)((word >> (kLocalBits * k)) & kLocalMask); }
+
+constexpr int kFusedThreads = kTileCells;
+constexpr size_t kTileMaxLds = 64 * 1024;  // of one workgroup
+
+// Gathered per edge from memory, the cells and nodes took 65 gathers of ~26
+// lines per wave (the L1 busy 63 % of the time, its return path 91 %).
+// Staged in LDS, a tile reads its own cells and a copy of its nodes once,
+// coalesced, and gathers only the ~130 cells around it; every further use is
+// an LDS read by local index, and the tables shrink to one 16-byte record
+// per cell and 8 bytes per evaluation.  What bounds it now is the FP64 VALU
+// (75 % busy) and, before the first barrier, two levels of loads (the lists
+// are read at fixed strides so that they wait for nothing): 40.5 KB of LDS
+// for a Delaunay mesh's 256-cell tile, so four workgroups share a CU
+// (three, at 42.6 KB with F1 and F2 kept of every edge, took 255 us at 4M
+// cells; 240 cells per tile 221).  The edges that only the ring's draining
+// steps need come last and give their mass flux alone.  Us per launch,
+// gathering / staged, dam break: fused stage 283 / 219 (4M cells), 73.3 /
+// 62.1 (1M), 23.1 / 21.5 (250k); after the flux pass 164 / 139, 41.7 / 38.5,
+// 13.7 / 12.6; of 24 ensemble members (0.7M cells) 57.3 / 50.6 and 33.1 / 31.5.
 template <int FLUX, int WS, bool LEN, bool NT, bool FF>
 __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(DevMesh M, DevTiles P, DevState S, DevState U0,
                                                       DevOut O, DevWork W, StageArgs A, int64_t t0, int64_t t1,
                                                       int store) {
-  __shared__ double sF0[kTileMaxEval], sF1[kTileMaxEval], sF2[kTileMaxEval];
-  __shared__ double sD[kTileMaxLocal];
+  extern __shared__ double lds[];
   // the evaluating instance walks the tiles backwards (it follows a
   // forward reconstruction); the FF instance forwards (it follows k_flux)
   const int64_t tile = t0 + (FF ? logical_block() : logical_block_reversed());
   if (A.pw_clear && blockIdx.x == 0 && threadIdx.x == 0) *A.pw_clear = 0u;
   if (tile >= t1) return;  // padding workgroups of the XCD-aware grid
+  const TileHead h = P.head[tile];
   const int64_t c0 = tile * kTileCells;
   const int nc = (int)(M.T - c0 < kTileCells ? M.T - c0 : kTileCells);
-  const int rg0 = P.ring_off[tile], nr = P.ring_off[tile + 1] - rg0;
-  const int e0 = P.ev_off[tile], ne = P.ev_off[tile + 1] - e0;
   const int tid = threadIdx.x;
-  const int64_t T = M.T;
+  const int lc = kTileCells + P.sx;
+  double* const cw = lds;  // w0 of the local cells, then the draining steps
+  double* const cgx = cw + lc;
+  double* const cgy = cgx + lc;
+  double* const cu = cgy + lc;
+  double* const cv = cu + lc;
+  double* const ccx = cv + lc;
+  double* const ccy = ccx + lc;
+  double* const sD = lds;
+  const int ln = FF && !LEN ? P.lo : P.sn;
+  double* const nx_ = lds + (FF ? kTileCells + P.sr : 7 * lc);
+  double* const ny_ = nx_ + ln;
+  double* const nz_ = ny_ + ln;
+  double* const sF0 = nz_ + ln;
+  double* const sF1 = sF0 + P.se;
+  double* const sF2 = sF1 + P.la;
+  auto lnode = [&](int l) { return V3{nx_[l], ny_[l], nz_[l]}; };
+  const double* const tn = P.tnode + tile * 3 * P.sn;
+  const int* const xl = P.xcell + tile * P.sx;
 
-  // ---- edge fluxes (k_flux's operations), one evaluation per LDS slot;
-  // the edge record gives both cells and nodes (one load level, as the
-  // separate flux kernel's edge tables)
-  // index loads of the later phases, issued before the flux phase: the
-  // own cell's slot codes, flags and vertex ids, and the thread's ring
-  // entry (nl <= kTileMaxLocal = 2 kTileCells <= kTileCells + kFusedThreads:
-  // at most one per thread)
+  // Every load that waits for no other comes first: the cells around the
+  // tile by number, its nodes, its own cells.
   const bool mine = tid < nc;
   const int i = (int)(c0 + (mine ? tid : 0));
-  uint32_t code[3];
-#pragma unroll
-  for (int k = 0; k < 3; ++k) code[k] = P.code[k * T + i];
-  const CVtx cvi = M.cv[i];
-  const int tpi[3] = {cvi.v0, cvi.v1, cvi.v2};
-  const uint32_t fli = cvi.fl;
-  const int nl = kTileCells + nr;
-  const int lr = kTileCells + tid;
-  int xr = 0;
-  uint32_t cdr[3] = {0u, 0u, 0u};
-  if (lr < nl) {
-    xr = P.ring_cell[rg0 + tid];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) cdr[k] = P.ring_code[3 * (rg0 + tid) + k];
-  }
-
-  // the own cell's update and draining inputs, and the ring cell's
-  // draining inputs (loaded before the flux phase by the FF instance, whose
-  // flux phase is loads only; after it by the evaluating one, whose flux
-  // phase needs the registers)
-  RhsCell q;
-  double w, u, v, w0 = 0., u0 = 0., v0 = 0.;
   const bool comb = A.a0 != 0.;
-  auto load_own = [&]() {
-    q.fl = fli;
-    q.mu = load_muscl(S, W, i);
-    q.wi = S.w[S.at(i)];
-    q.p[0] = node(M, tpi[0]);
-    q.p[1] = node(M, tpi[1]);
-    q.p[2] = node(M, tpi[2]);
-    w = S.w[S.at(i)];
-    u = S.u[S.at(i)];
-    v = S.v[S.at(i)];
-    if (comb) {
-      w0 = U0.w[U0.at(i)];
-      u0 = U0.u[U0.at(i)];
-      v0 = U0.v[U0.at(i)];
-    }
-  };
-  double hr = 0., arear = 0.;
-  uint32_t flr = 0u;
-  V3 rp0{0., 0., 0.}, rp1{0., 0., 0.}, rp2{0., 0., 0.};
-  auto load_ring = [&]() {
-    if (lr < nl) {
-      const CVtx cvr = M.cv[xr];
-      if (LEN) {
-        rp0 = node(M, cvr.v0);
-        rp1 = node(M, cvr.v1);
-        rp2 = node(M, cvr.v2);
-      }
-      hr = S.w[S.at(xr)] - M.bc[xr];
-      flr = cvr.fl;
-      arear = M.area[xr];
-    }
-  };
+  const int xc = tid < (FF ? P.sr : P.sx) ? xl[tid] : i;
+  const TileCell tc = P.cell[i];
+  V3 nd{0., 0., 0.};
+  if (tid < ln) nd = V3{tn[tid], tn[P.sn + tid], tn[2 * P.sn + tid]};
+  const bool ringed = tid < h.nr;  // the ring cell whose draining step this thread takes (nr <= kTileCells)
+  RingCode rc{0u, 0u};
+  double rbc = 0., arear = 0., hr = 0.;
+  if (ringed) {
+    rc = P.xcode[tile * P.sr + tid];
+    const double* const r = P.tring + 2 * (tile * P.sr + tid);
+    rbc = r[0];
+    arear = r[1];
+  }
+  RhsCell q;
+  q.mu = load_muscl(S, W, i);
+  double w, u, v, w0 = 0., u0 = 0., v0 = 0.;
+  w = S.w[S.at(i)];
+  u = S.u[S.at(i)];
+  v = S.v[S.at(i)];
+  if (comb) {
+    w0 = U0.w[U0.at(i)];
+    u0 = U0.u[U0.at(i)];
+    v0 = U0.v[U0.at(i)];
+  }
+  const int nn = FF && !LEN ? h.nn0 : h.nn;
   if constexpr (FF) {
-    load_own();
-    load_ring();
     // fluxes of the stage's flux pass, written by the separate flux kernel;
     // ne <= kTileMaxEval: at most kFE evaluations per thread, every load of
     // them issued before the first LDS write
@@ -139,97 +138,154 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
 #pragma unroll
     for (int it = 0; it < kFE; ++it) {
       const int j = tid + it * kFusedThreads;
-      ev[it] = j < ne ? P.evedge[e0 + j] : -1;
+      ev[it] = j < P.se ? P.evedge[tile * P.se + j] : 0;
     }
+    if (ringed) hr = S.w[S.at(xc)] - rbc;
     double f0[kFE], f1[kFE], f2[kFE];
 #pragma unroll
     for (int it = 0; it < kFE; ++it) {
-      const int e = ev[it] < 0 ? 0 : ev[it];
-      f0[it] = W.f0[e];
-      f1[it] = W.f1[e];
-      f2[it] = W.f2[e];
+      f0[it] = W.f0[ev[it]];
+      if (tid + it * kFusedThreads < h.na) {
+        f1[it] = W.f1[ev[it]];
+        f2[it] = W.f2[ev[it]];
+      }
     }
 #pragma unroll
     for (int it = 0; it < kFE; ++it) {
       const int j = tid + it * kFusedThreads;
-      if (j < ne) {
-        sF0[j] = f0[it];
+      if (j < h.ne) sF0[j] = f0[it];
+      if (j < h.na) {
         sF1[j] = f1[it];
         sF2[j] = f2[it];
       }
     }
   } else {
-    // the next evaluation's edge record is loaded before this one's gathers
-    EdgeRec rn = tid < ne ? P.evrec[e0 + tid] : EdgeRec{0, 0, 0, 0};
-    for (int j = tid; j < ne; j += kFusedThreads) {
-      const EdgeRec r = rn;
-      if (j + kFusedThreads < ne) rn = P.evrec[e0 + j + kFusedThreads];
-      const int f = r.et0, t = r.et1;
-      const int tr = t < 0 ? f : t;  // boundary edges read their own cell twice: R = L
-      const V3 Pa = node(M, r.ep0), Pb = node(M, r.ep1);
-      const Muscl mf = load_muscl(S, W, f), mt = load_muscl(S, W, tr);
-      const CXY cf = M.cxy[f], ct = M.cxy[tr];
-      const double cxf = cf.x, cyf = cf.y, cxt = ct.x, cyt = ct.y;
-      const double hf = (t == kSolidWall && !M.eb) ? S.w[S.at(f)] - M.bc[f] : 0.;
-      const double le = edge_len(Pa, Pb);
+    auto stage_cell = [&](int l, const Muscl& m, double cx, double cy) {
+      cw[l] = m.w0;
+      cgx[l] = m.gx;
+      cgy[l] = m.gy;
+      cu[l] = m.u0;
+      cv[l] = m.v0;
+      ccx[l] = cx;
+      ccy[l] = cy;
+    };
+    const double* const xo = P.txc + 2 * tile * P.sx;
+    if (tid < h.nx) {
+      const Muscl m = load_muscl(S, W, xc);
+      if (ringed) hr = S.w[S.at(xc)] - rbc;
+      stage_cell(kTileCells + tid, m, xo[2 * tid], xo[2 * tid + 1]);
+    }
+    for (int j = tid + kFusedThreads; j < h.nx; j += kFusedThreads)
+      stage_cell(kTileCells + j, load_muscl(S, W, xl[j]), xo[2 * j], xo[2 * j + 1]);
+  }
+  if (tid < nn) {
+    nx_[tid] = nd.x;
+    ny_[tid] = nd.y;
+    nz_[tid] = nd.z;
+  }
+  for (int j = tid + kFusedThreads; j < nn; j += kFusedThreads) {
+    nx_[j] = tn[j];
+    ny_[j] = tn[P.sn + j];
+    nz_[j] = tn[2 * P.sn + j];
+  }
+  const EvalCode* const evl = P.ev + tile * P.se;
+  EvalCode rn{0u, 0u};
+  if (!FF && tid < P.se) rn = evl[tid];
+  __syncthreads();
+  if constexpr (!FF) {
+    if (mine) {  // the centroid as the setup kernel computes M.cxy
+      const V3 c = centroid(lnode(local3(tc.nodes, 0)), lnode(local3(tc.nodes, 1)), lnode(local3(tc.nodes, 2)));
+      cw[tid] = q.mu.w0;
+      cgx[tid] = q.mu.gx;
+      cgy[tid] = q.mu.gy;
+      cu[tid] = q.mu.u0;
+      cv[tid] = q.mu.v0;
+      ccx[tid] = c.x;
+      ccy[tid] = c.y;
+    }
+    __syncthreads();
+    // ---- edge fluxes (k_flux's operations), one evaluation per LDS slot;
+    // the next evaluation's code is loaded before this one's arithmetic
+    auto lmuscl = [&](int l) { return Muscl{cw[l], cgx[l], cgy[l], cu[l], cv[l]}; };
+    for (int j = tid; j < h.ne; j += kFusedThreads) {
+      const EvalCode r = rn;
+      if (j + kFusedThreads < h.ne) rn = evl[j + kFusedThreads];
+      const int f = local3(r.cells, 0), t = local3(r.cells, 1);
+      const bool wall = t == (int)kLocalWall;
+      const bool all = j < h.na;
+      const int tr = t >= (int)kLocalMax ? f : t;  // boundary edges read their own cell twice: R = L
+      const V3 Pa = lnode(local3(r.nodes, 0)), Pb = lnode(local3(r.nodes, 1));
+      const Muscl mf = lmuscl(f);
+      const double cxf = ccx[f], cyf = ccy[f];
       const V3 E = midpoint(Pa, Pb);
-      double tx, ty;
-      tangent(Pa, Pb, le, V3{cxf, cyf, 0.}, tx, ty);
+      double le, tx, ty;
+      PlainGeometry::edge(Pa, Pb, V3{cxf, cyf, 0.}, le, tx, ty);
       const double nx = ty, ny = -tx;
       double F[3];
       double lw = 1.0;  // the CFL candidate is not taken here (unused)
-      if (t == kSolidWall) {
-        // SWE_OPT_EXACT_BALANCE: the inside edge depth instead of the cell mean
-        const double hw = M.eb ? slot_value(mf, cxf, cyf, E).w - E.z : hf;
+      if (wall) {
+        // the cell average; SWE_OPT_EXACT_BALANCE: the inside edge depth
+        double hw;
+        if (M.eb) {
+          hw = slot_value(mf, cxf, cyf, E).w - E.z;
+        } else {
+          const int g = f < kTileCells ? (int)c0 + f : xl[f - kTileCells];
+          hw = S.w[S.at(g)] - M.bc[g];
+        }
         elem_flux(nx, ny, hw, 0., 0., F[0], F[1], F[2]);
       } else {
         const Slot L = slot_value(mf, cxf, cyf, E);
-        const Slot R = slot_value(mt, cxt, cyt, E);
-        if (FLUX == 0) flux_hll<WS>(nx, ny, E.z, L, R, 1.0, A.cor, lw, F, M.eb != 0);
-        else flux_hllc<WS>(tx, ty, E.z, L, R, 1.0, A.cor, lw, F, M.eb != 0);
+        const Slot R = slot_value(lmuscl(tr), ccx[tr], ccy[tr], E);
+        if (FLUX == 0) flux_hll<WS>(nx, ny, E.z, L, R, 1.0, A.cor, lw, F, M.eb != 0, all);
+        else flux_hllc<WS>(tx, ty, E.z, L, R, 1.0, A.cor, lw, F, M.eb != 0, all);
       }
       sF0[j] = F[0];
-      sF1[j] = F[1];
-      sF2[j] = F[2];
-      if (store && f >= c0 && f < c0 + nc) {  // the edge's one owning evaluation: its et0 cell is ours
-        const int e = P.evedge[e0 + j];
+      if (all) {
+        sF1[j] = F[1];
+        sF2[j] = F[2];
+      }
+      if (store && j < h.ne0) {  // the edge's one owning evaluation: its et0 cell is ours
+        const int e = P.evedge[tile * P.se + j];
         out_store<NT>(&W.f0[e], F[0]);
         out_store<NT>(&W.f1[e], F[1]);
         out_store<NT>(&W.f2[e], F[2]);
       }
     }
+    __syncthreads();
+    q.mu = lmuscl(tid);  // read before the draining steps take w0's place
   }
-  __syncthreads();
 
-  // ---- draining time steps of every local cell (k_drain's operations).
-  // The thread's own cell (tid < nc) is also the cell it updates: its
-  // update inputs are loaded here with its draining inputs, so one latency
-  // covers both phases' loads.
-  if constexpr (!FF) load_own();
-  // the draining step of a cell from its depth, edges and flux slots
-  auto drain_dt = [&](double h, uint32_t fl, const uint32_t* cd, const V3& p0, const V3& p1, const V3& p2,
-                      double area) -> double {
-    if (!is_wet(h)) return 0.;
+  // ---- draining time steps of every local cell (k_drain's operations)
+  auto drain_dt = [&](double hh, uint32_t slots, uint32_t fl, double area) -> double {
+    if (!is_wet(hh)) return 0.;
     double sum = 0.;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const double fe = sF0[cd[k] >> 16];
+      const int s = local3(slots, k);
+      const double fe = sF0[s];
       double out = sgn_pos(fl, k) ? fe : -fe;
-      if (LEN) out = out * edge_len(pick(p0, p1, p2, ep0_local(fl, k)), pick(p0, p1, p2, ep1_local(fl, k)));
+      if (LEN) {
+        const uint32_t en = evl[s].nodes;
+        out = out * edge_len(lnode(local3(en, 0)), lnode(local3(en, 1)));
+      }
       sum += dmax(0., out);
     }
-    return sum > kTol ? area * h / sum : INFINITY;
+    return sum > kTol ? area * hh / sum : INFINITY;
   };
+  q.fl = tc.flags;
+  q.wi = w;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) q.p[k] = mine ? lnode(local3(tc.nodes, k)) : V3{0., 0., 0.};
+  const double bc = centroid(q.p[0], q.p[1], q.p[2]).z;
   if (mine) {
     // the centroid bathymetry and area from the vertices, as the setup
     // kernel computes M.bc and M.area (the same functions: the same bits)
-    const double d = drain_dt(w - centroid(q.p[0], q.p[1], q.p[2]).z, q.fl, code, q.p[0], q.p[1], q.p[2],
-                              tri_area(q.p[0], q.p[1], q.p[2]));
+    const double d = drain_dt(w - bc, tc.slots, tc.flags, tri_area(q.p[0], q.p[1], q.p[2]));
     sD[tid] = d;
+    q.dti = d;
     if (store) out_store<NT>(&W.dtd[i], d);
   }
-  if constexpr (!FF) load_ring();
-  if (lr < nl) sD[lr] = drain_dt(hr, flr, cdr, rp0, rp1, rp2, arear);
+  if (ringed) sD[kTileCells + tid] = drain_dt(hr, rc.slots, rc.flags, arear);
   __syncthreads();
 
   // ---- update of the tile's cells (k_update's operations; the fluxes and
@@ -251,18 +307,19 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
     }
     dts = A.coef * member_dt(M, A, inst);
   }
-  q.dti = sD[tid];
-  const double bc = centroid(q.p[0], q.p[1], q.p[2]).z;
   double R0, R1, R2;
-  rhs_compute_by(
+  rhs_compute_by<PlainGeometry>(
       q,
       [&](int k, double& F0, double& F1, double& F2, double& dtik) {
-        const int s = (int)(code[k] >> 16);
-        const uint32_t nb = code[k] & 0xffffu;
+        const int s = local3(tc.slots, k), nb = local3(tc.nbs, k);
         F0 = sF0[s];
         F1 = sF1[s];
         F2 = sF2[s];
-        dtik = nb >= kNbOut ? INFINITY : sD[nb];
+        dtik = nb >= (int)kLocalMax ? INFINITY : sD[nb];
+      },
+      [&](int k, V3& Pa, V3& Pb) {
+        Pa = lnode((int)((tc.nodes >> (kLocalBits * (uint32_t)ep0_local(tc.flags, k))) & kLocalMask));
+        Pb = lnode((int)((tc.nodes >> (kLocalBits * (uint32_t)ep1_local(tc.flags, k))) & kLocalMask));
       },
       dts, A.cor, A.fric, M.eb != 0, R0, R1, R2);
   const double hh = w - bc;
@@ -287,6 +344,37 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
   out_store<NT>(&O.v[O.at(i)], ov);
 }
 
+// the tiles' copies of the static geometry, one workgroup per tile
+__global__ void __launch_bounds__(256) k_setup_tiles(DevMesh M, DevTiles P) {
+  const int64_t t = blockIdx.x;
+  for (int j = threadIdx.x; j < P.sn; j += 256) {
+    const NodeRec r = M.pn[P.node[t * P.sn + j]];
+    double* const o = P.tnode + t * 3 * P.sn + j;
+    o[0] = r.x;
+    o[P.sn] = r.y;
+    o[2 * P.sn] = r.z;
+  }
+  for (int j = threadIdx.x; j < P.sx; j += 256) {
+    const int x = P.xcell[t * P.sx + j];
+    const CXY c = M.cxy[x];
+    P.txc[2 * (t * P.sx + j)] = c.x;
+    P.txc[2 * (t * P.sx + j) + 1] = c.y;
+    if (j < P.sr) {
+      P.tring[2 * (t * P.sr + j)] = M.bc[x];
+      P.tring[2 * (t * P.sr + j) + 1] = M.area[x];
+    }
+  }
+}
+hipError_t launch_setup_tiles(const DevMesh& M, const DevTiles& P, hipStream_t st) {
+  if (P.ntiles > 0) hipLaunchKernelGGL(k_setup_tiles, dim3((unsigned)P.ntiles), dim3(256), 0, st, M, P);
+  return hipGetLastError();
+}
+
+bool fused_fits(const DevTiles& P) {
+  return sizeof(double) * (size_t)lds_doubles(P, false, true) <= kTileMaxLds &&
+         sizeof(double) * (size_t)lds_doubles(P, true, true) <= kTileMaxLds;
+}
+
 hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, const DevState& U0,
                         const DevOut& O, const DevWork& W, const StageArgs& A, int flux, int ws, int opts,
                         hipStream_t st, bool store, bool from_fluxes) {
@@ -299,19 +387,20 @@ hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, 
   const dim3 g = grid_for_bs(t1 - t0, 1), b(kFusedThreads);
   const bool len = (opts & kOptDrainLength) != 0;
   const int sto = store ? 1 : 0;
+  const unsigned lds = (unsigned)(sizeof(double) * (size_t)lds_doubles(P, from_fluxes, len));
   if (from_fluxes) {  // the flux scheme does not enter: one instance per drain / store variant
-    if (len && M.nt) hipLaunchKernelGGL((k_fused<0, 0, true, true, true>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else if (len) hipLaunchKernelGGL((k_fused<0, 0, true, false, true>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else if (M.nt) hipLaunchKernelGGL((k_fused<0, 0, false, true, true>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else hipLaunchKernelGGL((k_fused<0, 0, false, false, true>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    if (len && M.nt) hipLaunchKernelGGL((k_fused<0, 0, true, true, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else if (len) hipLaunchKernelGGL((k_fused<0, 0, true, false, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else if (M.nt) hipLaunchKernelGGL((k_fused<0, 0, false, true, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else hipLaunchKernelGGL((k_fused<0, 0, false, false, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
     return hipGetLastError();
   }
 #define SWE_FUSED(F, Wv)                                                                             \
   if (flux == F && ws == Wv) {                                                                       \
-    if (len && M.nt) hipLaunchKernelGGL((k_fused<F, Wv, true, true, false>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);   \
-    else if (len) hipLaunchKernelGGL((k_fused<F, Wv, true, false, false>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);     \
-    else if (M.nt) hipLaunchKernelGGL((k_fused<F, Wv, false, true, false>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);    \
-    else hipLaunchKernelGGL((k_fused<F, Wv, false, false, false>), g, b, 0, st, M, P, S, U0, O, W, A, t0, t1, sto);             \
+    if (len && M.nt) hipLaunchKernelGGL((k_fused<F, Wv, true, true, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);   \
+    else if (len) hipLaunchKernelGGL((k_fused<F, Wv, true, false, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);     \
+    else if (M.nt) hipLaunchKernelGGL((k_fused<F, Wv, false, true, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);    \
+    else hipLaunchKernelGGL((k_fused<F, Wv, false, false, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);             \
     return hipGetLastError();                                                                        \
   }
   SWE_FUSED(0, 0) SWE_FUSED(0, 1) SWE_FUSED(0, 2) SWE_FUSED(1, 0) SWE_FUSED(1, 1) SWE_FUSED(1, 2)

@@ -318,6 +318,10 @@ hipError_t launch_adjoint_finish(const DevMesh& M, const DevAdj& J, double* zbar
 // from_fluxes the stage's fluxes are already in W (the separate flux pass
 // of a CFL step's first stage) and are read instead of evaluated.
 struct DevTiles;
+// the tiles' data fits the stage kernels' LDS
+bool fused_fits(const DevTiles& P);
+// the tiles' copies of the static geometry, after launch_setup_geometry
+hipError_t launch_setup_tiles(const DevMesh& M, const DevTiles& P, hipStream_t st);
 hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, const DevState& U0,
                         const DevOut& O, const DevWork& W, const StageArgs& A, int flux, int ws, int opts,
                         hipStream_t st, bool store = false, bool from_fluxes = false);

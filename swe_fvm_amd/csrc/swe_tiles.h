@@ -41,15 +41,80 @@ struct TileTables {
 bool build_tiles(int64_t T, const int* tt, const int* te, const uint32_t* cflag, const int* et0, const int* et1,
                  const int* ep0, const int* ep1, TileTables& out);
 
+// The stage kernels' view of the tiles: a tile keeps the data of its cells,
+// of the ring and of the cells beyond the ring (the other side of the ring
+// cells' outer edges), and of the nodes of every evaluated edge in LDS, and
+// the tables name them by local index: cells 0 .. kTileCells - 1 the tile's
+// own, then the ring, then the cells beyond; nodes those of the tile's own
+// cells first.  Indices take 10 bits.
+constexpr uint32_t kLocalBits = 10, kLocalMask = (1u << kLocalBits) - 1u;
+constexpr uint32_t kLocalWall = kLocalMask, kLocalFree = kLocalMask - 1u;  // in the place of a neighbour
+constexpr uint32_t kLocalMax = kLocalFree;  // local indices are below
+// Every list of a tile starts at tile * stride (the longest of any tile), so
+// that its loads wait for nothing but the tile's number; entries past a
+// tile's counts hold valid indices.
+struct alignas(16) TileHead {
+  uint16_t nr, nx;   // ring cells; ring and beyond
+  uint16_t nn0, nn;  // nodes of the own cells; all
+  // evaluations: of edges the tile owns (et0 is its cell), which come first;
+  // of all edges of its cells, which come before those the ring alone has (a
+  // draining step needs the mass flux only); all
+  uint16_t ne0, na, ne;
+  uint16_t pad;
+};
+// three local indices per word: vertices, neighbours across edge k (or
+// kLocalWall / kLocalFree), flux slots of edge k; and the cell's flags
+struct alignas(16) TileCell {
+  uint32_t nodes, nbs, slots, flags;
+};
+struct alignas(8) RingCode {
+  uint32_t slots, flags;
+};
+// an evaluation: local cells et0 | et1 << 10 (or a boundary code), local
+// nodes ep0 | ep1 << 10
+struct alignas(8) EvalCode {
+  uint32_t cells, nodes;
+};
+struct StageTables {
+  int64_t ntiles = 0;
+  std::vector<TileHead> head;
+  std::vector<TileCell> cell;   // [T]
+  int sx = 0, sr = 0, sn = 0, se = 0;  // strides: the largest nx, nr, nn, ne
+  int max_own_nodes = 0, max_own_ev = 0;  // the largest nn0, na
+  std::vector<int> xcell;       // [tile][sx] global ids of ring and beyond
+  std::vector<RingCode> xcode;  // [tile][sr] of the ring cells
+  std::vector<int> node;        // [tile][sn] global node ids
+  std::vector<EvalCode> ev;     // [tile][se]
+  std::vector<int> evedge;      // [tile][se] the edge of each evaluation
+};
+// build_tiles' tables in this form, built by several threads; false where
+// build_tiles refuses the mesh or a local index does not fit
+bool build_stage_tables(int64_t T, const int* tp, const int* tt, const int* te, const uint32_t* cflag, const int* et0,
+                        const int* et1, const int* ep0, const int* ep1, StageTables& out);
+
+// whether the edges' geometry needs none of the special cases of the IEEE
+// square root and division (PlainGeometry): every edge's coordinate
+// differences are +0 or of magnitude 2^-400 .. 2^400, not both 0, and no
+// coordinate is a negative zero or not finite
+bool plain_geometry(int64_t V, const double* px, const double* py, int64_t E, const int* ep0, const int* ep1);
+
 struct DevTiles {
-  const uint32_t* code;
-  const int* ring_off;
-  const int* ring_cell;
-  const uint32_t* ring_code;
-  const int* ev_off;
-  const EdgeRec* evrec;  // et0, et1, ep0, ep1 of each evaluated edge
-  const int* evedge;     // the edge of each evaluation (for the fluxes a storing launch writes)
+  const TileHead* head;
+  const TileCell* cell;
+  const int* xcell;
+  const RingCode* xcode;
+  const int* node;
+  const EvalCode* ev;
+  const int* evedge;
+  // static geometry in the tiles' order (the setup kernels): node
+  // coordinates [tile][3][sn], centroids [tile][sx][2] of ring and beyond,
+  // bathymetry and area [tile][sr][2] of the ring
+  double* tnode;
+  double* txc;
+  double* tring;
   int64_t ntiles;
+  int sx, sr, sn, se;  // strides
+  int lo, la;          // the most nodes of a tile's own cells, evaluations of its cells' edges
 };
 
 }  // namespace swe
