@@ -498,20 +498,27 @@ void swe_destroy(swe_solver* s) {  // teardown: failures cannot be reported
   delete s;
 }
 
-// the host image of a state allocation in the solver's layout (padding cells
-// zero) from / to the caller's (T, 3) primitive array
+// A state buffer that holds nothing anyone will read: not the current state,
+// not the input of a fused stage whose fluxes are still to be recomputed,
+// and for ensembles not the buffer an Euler step writes next, where finished
+// members keep their state.
+static int free_buffer(const swe_solver* s) {
+  for (int b = 0; b < 3; ++b) {
+    if (b == s->cur || (s->flux_stale && b == s->stale_in)) continue;
+    if (s->n_inst > 0 && b == (s->cur == 0 ? 1 : 0)) continue;
+    return b;
+  }
+  return -1;  // not reached: at most two of the three are taken
+}
+
+// The caller's (T, 3) primitive array crosses through a free state buffer
+// and is turned into the solver's layout (padding cells zero) on the device.
 int swe_set_state(swe_solver* s, const double* prim) {
   if (!s || !prim) return fail(SWE_ERR_ARG, "null argument");
   if (int rc = set_device(s)) return rc;
-  std::vector<double> h(size_t(3 * s->Tpad), 0.);
-  const uint32_t mask = layout_mask(s->lay_b);
-  const int64_t d = layout_plane(s);
-  for (int64_t i = 0; i < s->T; ++i) {
-    const int64_t a = state_at(i, mask);
-    h[size_t(a)] = prim[3 * i]; h[size_t(d + a)] = prim[3 * i + 1]; h[size_t(2 * d + a)] = prim[3 * i + 2];
-  }
-  SWE_CHECK(hipMemcpyAsync(s->sbuf[s->cur], h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, s->stream),
-            "hipMemcpy");
+  double* const rows = s->sbuf[free_buffer(s)];
+  SWE_CHECK(hipMemcpyAsync(rows, prim, sizeof(double) * size_t(3 * s->T), hipMemcpyHostToDevice, s->stream), "hipMemcpy");
+  SWE_CHECK(launch_rows_in(rows, out_of(s, s->cur), s->T, s->Tpad, s->stream), "rows_in");
   SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
   return SWE_OK;
 }
@@ -519,16 +526,10 @@ int swe_set_state(swe_solver* s, const double* prim) {
 int swe_get_state(swe_solver* s, double* prim) {
   if (!s || !prim) return fail(SWE_ERR_ARG, "null argument");
   if (int rc = set_device(s)) return rc;
-  std::vector<double> h(size_t(3 * s->Tpad));
-  SWE_CHECK(hipMemcpyAsync(h.data(), s->sbuf[s->cur], sizeof(double) * h.size(), hipMemcpyDeviceToHost, s->stream),
-            "hipMemcpy");
+  double* const rows = s->sbuf[free_buffer(s)];
+  SWE_CHECK(launch_rows_out(state_of(s, s->cur), rows, s->T, s->stream), "rows_out");
+  SWE_CHECK(hipMemcpyAsync(prim, rows, sizeof(double) * size_t(3 * s->T), hipMemcpyDeviceToHost, s->stream), "hipMemcpy");
   SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
-  const uint32_t mask = layout_mask(s->lay_b);
-  const int64_t d = layout_plane(s);
-  for (int64_t i = 0; i < s->T; ++i) {
-    const int64_t a = state_at(i, mask);
-    prim[3 * i] = h[size_t(a)]; prim[3 * i + 1] = h[size_t(d + a)]; prim[3 * i + 2] = h[size_t(2 * d + a)];
-  }
   return SWE_OK;
 }
 
@@ -1583,10 +1584,8 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
     rc = dev_fail(e, "copy");
   tm.mark(1, s->stream);
   if (!rc) {
-    std::vector<double> h(static_cast<size_t>(3 * T));
-    for (int64_t i = 0; i < T; ++i)
-      for (int q = 0; q < 3; ++q) h[size_t(q * T + i)] = final_bar[3 * i + q];
-    if ((e = hipMemcpyAsync(bar_a, h.data(), size_t(S3), hipMemcpyHostToDevice, s->stream)) != hipSuccess ||
+    if ((e = hipMemcpyAsync(bar_b, final_bar, size_t(S3), hipMemcpyHostToDevice, s->stream)) != hipSuccess ||
+        (e = launch_rows_in(bar_b, out3(Buf3{bar_a}, T), T, T, s->stream)) != hipSuccess ||
         (e = hipMemsetAsync(J.zc, 0, sizeof(double) * size_t(3 * T), s->stream)) != hipSuccess ||
         (e = hipMemsetAsync(J.p1bar, 0, sizeof(double) * size_t(3 * T), s->stream)) != hipSuccess ||
         (e = hipMemsetAsync(J.zn_acc, 0, sizeof(double) * size_t(std::max<int64_t>(V, 1)), s->stream)) != hipSuccess ||
@@ -1680,14 +1679,12 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
     rc = dev_fail(e, "adjoint finish");
   tm.mark(2, s->stream);
   if (!rc) {
-    std::vector<double> h(static_cast<size_t>(3 * T));
-    if ((e = hipMemcpyAsync(h.data(), ob, size_t(S3), hipMemcpyDeviceToHost, s->stream)) != hipSuccess ||
+    if ((e = launch_rows_out(st3(Buf3{ob}, T), sb, T, s->stream)) != hipSuccess ||
+        (e = hipMemcpyAsync(state0_bar, sb, size_t(S3), hipMemcpyDeviceToHost, s->stream)) != hipSuccess ||
         (z_bar && (e = hipMemcpyAsync(z_bar, zb, sizeof(double) * size_t(V), hipMemcpyDeviceToHost, s->stream)) != hipSuccess) ||
         (e = hipStreamSynchronize(s->stream)) != hipSuccess) {
       rc = dev_fail(e, "adjoint download");
     } else {
-      for (int64_t i = 0; i < T; ++i)
-        for (int q = 0; q < 3; ++q) state0_bar[3 * i + q] = h[size_t(q * T + i)];
       if (ms) {
         ms[0] = tm.ms(0, 1);
         ms[1] = tm.ms(1, 2);
@@ -1752,14 +1749,12 @@ int swe_tangent_run(swe_solver* s, int scheme, double dt, const double* dts, int
   Q.f2 = q; q += E;
   auto tst = [&](int k) { return DevState{td[k], td[k] + T, td[k] + 2 * T}; };
   auto tout = [&](int k) { return DevOut{td[k], td[k] + T, td[k] + 2 * T}; };
-  std::vector<double> h(static_cast<size_t>(3 * T));
-  for (int64_t i = 0; i < T; ++i)
-    for (int c = 0; c < 3; ++c) h[size_t(c * T + i)] = state0_dot[3 * i + c];
   std::vector<double> hz(static_cast<size_t>(std::max<int64_t>(V, 1)), 0.);
   if (z_dot) std::copy(z_dot, z_dot + V, hz.begin());
   int rc = SWE_OK;
-  hipError_t e = hipMemcpyAsync(td[s->cur], h.data(), sizeof(double) * size_t(3 * T), hipMemcpyHostToDevice,
-                                s->stream);
+  hipError_t e = hipMemcpyAsync(td[(s->cur + 1) % 3], state0_dot, sizeof(double) * size_t(3 * T),
+                                hipMemcpyHostToDevice, s->stream);
+  if (e == hipSuccess) e = launch_rows_in(td[(s->cur + 1) % 3], tout(s->cur), T, T, s->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(zd, hz.data(), sizeof(double) * size_t(V), hipMemcpyHostToDevice, s->stream);
   StageCoef sc[3];
   const int ns = stage_list(scheme, sc);
@@ -1779,13 +1774,13 @@ int swe_tangent_run(swe_solver* s, int scheme, double dt, const double* dts, int
     s->cur = ns == 1 ? b : a;
   }
   tm.mark(1, s->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(h.data(), td[s->cur], sizeof(double) * size_t(3 * T), hipMemcpyDeviceToHost, s->stream);
+  if (e == hipSuccess) e = launch_rows_out(tst(s->cur), td[(s->cur + 1) % 3], T, s->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(final_dot, td[(s->cur + 1) % 3], sizeof(double) * size_t(3 * T), hipMemcpyDeviceToHost, s->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
   if (e != hipSuccess) {
     rc = dev_fail(e, "tangent run");
   } else {
-    for (int64_t i = 0; i < T; ++i)
-      for (int c = 0; c < 3; ++c) final_dot[3 * i + c] = h[size_t(c * T + i)];
     if (ms) *ms = tm.ms(0, 1);
   }
   (void)hipStreamSynchronize(s->stream);  // cleanup: errors were reported above

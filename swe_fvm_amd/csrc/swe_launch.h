@@ -239,6 +239,10 @@ struct StageArgs {
 
 // the state of cells [0, T) rewritten from S's layout into O's
 hipError_t launch_relayout(const DevState& S, const DevOut& O, int64_t T, hipStream_t st);
+// cells [0, T) between a (T, 3) row-major array (w, u, v per cell) and O's or
+// S's layout; cells [T, Tpad) of O are set to zero
+hipError_t launch_rows_in(const double* rows, const DevOut& O, int64_t T, int64_t Tpad, hipStream_t st);
+hipError_t launch_rows_out(const DevState& S, double* rows, int64_t T, hipStream_t st);
 hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStream_t st);
 // zero_count false: W.pw_count is zero already (the stage before cleared it,
 // or launch_slot_counts); r (may be null): set to 1, for the flux pass that
