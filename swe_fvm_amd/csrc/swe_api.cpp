@@ -137,13 +137,16 @@ int materialize_fluxes(swe_solver* s) {
   return SWE_OK;
 }
 
+// the tiles the step's kernels take, null where they take none
+const DevTiles* tiles_of(const swe_solver* s) { return s->fused_ok && s->fused_on ? &s->tiles : nullptr; }
+
 // Both passes of the reconstruction of S into W; r: see launch_recon1.  W's
 // list is left in use: a stage whose last kernel clears it (pw_clear) sets
 // pw_clean again.
 hipError_t reconstruct(swe_solver* s, const DevState& S, unsigned long long* r = nullptr) {
   const bool clean = s->pw_clean;
   s->pw_clean = false;
-  hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, r);
+  hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, r, tiles_of(s));
   if (e == hipSuccess) e = launch_recon2(s->M, S, s->W, s->opts, s->stream);
   return e;
 }
@@ -1034,7 +1037,8 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
         const bool clean = s->pw_clean, fuse = use_fused(s, dt, st);
         s->pw_clean = false;
         timed(0, [&] {
-          return launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, fuse ? nullptr : s->rbits + st);
+          return launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, fuse ? nullptr : s->rbits + st,
+                               tiles_of(s));
         });
         timed(1, [&] { return launch_recon2(s->M, S, s->W, s->opts, s->stream); });
         if (fuse) {
@@ -1281,7 +1285,7 @@ int swe_autotune_layout(swe_solver* s, int reps, int* block, double* cost_ms) {
     const DevOut O = out_of(s, (s->cur + 1) % 3);
     const StageArgs A{0., 0., 1., 1e-6, 0., s->cor, rslot, nullptr, friction(s)};
     auto sep = [&]() -> hipError_t {
-      hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream);
+      hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream, true, nullptr, tiles_of(s));
       if (e == hipSuccess) e = launch_recon2(s->M, S, s->W, s->opts, s->stream);
       if (e == hipSuccess)
         e = launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, rslot, s->flux_items, s->flux_block, s->stream);
@@ -1292,7 +1296,7 @@ int swe_autotune_layout(swe_solver* s, int reps, int* block, double* cost_ms) {
       return e;
     };
     auto fus = [&]() -> hipError_t {
-      hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream);
+      hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream, true, nullptr, tiles_of(s));
       if (e == hipSuccess) e = launch_recon2(s->M, S, s->W, s->opts, s->stream);
       if (e == hipSuccess) e = launch_fused(s->M, s->tiles, S, S, O, s->W, A, s->flux, s->ws, s->opts, s->stream);
       return e;
@@ -1619,7 +1623,7 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
         else if (n + 1 < n1) O = out3(Buf3{seg + (m + 1) * 3 * T}, T);
         else O = g == nck - 1 ? out_of(s, (s->cur + 1) % 3) : out3(Buf3{sb}, T);  // U_N, or unused
         const DevWork Wq = slot_work(m * ns + q);
-        e = launch_recon1(s->M, Sq, Wq, s->opts, s->stream, false);
+        e = launch_recon1(s->M, Sq, Wq, s->opts, s->stream, false, nullptr, tiles_of(s));
         if (e == hipSuccess) e = launch_recon2(s->M, Sq, Wq, s->opts, s->stream);
         StageArgs A{sc[q].a0, sc[q].a1, sc[q].coef, dtn(n), 0., s->cor, s->rbits, nullptr, friction(s)};
         if (use_fused(s, dtn(n), q) && T < kFusedRecomputeMaxCells) {

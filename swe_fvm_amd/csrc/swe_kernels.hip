@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "swe_common.h"
+#include "swe_tiles.h"
 
 namespace swe {
 
@@ -135,6 +136,46 @@ __device__ __forceinline__ void fullwet_plane(const V3& p0, const V3& p1, const 
   }
   gx = tvd * gx;
   gy = tvd * gy;
+}
+
+// Pass 1's results of cell i of class k, and pass 2's work list (pw: the cell
+// goes in; every lane that is left must call this together).
+template <bool NT>
+__device__ __forceinline__ void recon_store(const DevWork& W, int i, int8_t k, double w0, double gx, double gy,
+                                            bool pw) {
+  // outputs read only by later kernels: out_store, nontemporal on large
+  // meshes, keeps L2 for the neighbour gathers (-1.5 % per step at 16M cells)
+  out_store<NT>(&W.mw[i], w0);
+  out_store<NT>(&W.mgx[i], gx);
+  out_store<NT>(&W.mgy[i], gy);
+  W.cls[i] = k;
+  // append partially wet cells to pass 2's work list, one atomic per wave
+  // (the order of the list is irrelevant: pass 2 is independent per cell).
+  // A level above every vertex (wet boundary cells) is pass 2's fallback to
+  // the pass-1 level already written: such cells are left out.
+  const unsigned long long m = __ballot(pw);
+  if (m) {
+    const int lane = threadIdx.x & 63;
+    const int leader = __ffsll((long long)m) - 1;
+    unsigned int base = 0;
+    if (lane == leader) base = atomicAdd(W.pw_count, (unsigned int)__popcll(m));
+    base = __shfl(base, leader, 64);
+    if (pw) {
+      const unsigned int below = __builtin_amdgcn_mbcnt_hi(
+          (unsigned int)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0u));
+      W.pw_list[base + below] = i;
+    }
+  }
+}
+
+// the PartWet1 levels of the n listed cells, one per lane of the workgroup
+__device__ __forceinline__ void level_list(const DevMesh& M, const DevState& S, const int* cell, double* lvl, int n) {
+  for (int q = threadIdx.x; q < n; q += kBlock) {
+    // b13 = zmax, b23 = zmin enter partwet1_w only through max / min
+    const int j = cell[q];
+    const CellRec r = M.crec[j];
+    lvl[q] = partwet1_w(r.zmin, r.zmin, r.zmax, r.bc, S.w[S.at(j)]);
+  }
 }
 
 // ---------------------------------------------------------------- pass 1 --
@@ -261,13 +302,7 @@ __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W
         sh.lev.cell[at[kk]] = jn[kk];
       }
     __syncthreads();
-    const int n = s_n;
-    for (int q = tid; q < n; q += kBlock) {
-      // b13 = zmax, b23 = zmin enter partwet1_w only through max / min
-      const int j = sh.lev.cell[q];
-      const CellRec r = M.crec[j];
-      sh.lev.lvl[q] = partwet1_w(r.zmin, r.zmin, r.zmax, r.bc, S.w[S.at(j)]);
-    }
+    level_list(M, S, sh.lev.cell, sh.lev.lvl, s_n);
     __syncthreads();
     if (own) w0 = sh.lev.lvl[at[0]];
 #pragma unroll
@@ -286,30 +321,161 @@ __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W
   } else if (!any_dry) {
     fullwet_plane<HEAD_GRAD>(p0, p1, p2, fl, w, cx, cy, wn, rn, nb, gx, gy);
   }
-  // outputs read only by later kernels: out_store, nontemporal on large
-  // meshes, keeps L2 for the neighbour gathers (-1.5 % per step at 16M cells)
-  out_store<NT>(&W.mw[i], w0);
-  out_store<NT>(&W.mgx[i], gx);
-  out_store<NT>(&W.mgy[i], gy);
-  W.cls[i] = k;
-  // append partially wet cells to pass 2's work list, one atomic per wave
-  // (the order of the list is irrelevant: pass 2 is independent per cell).
-  // A level above every vertex (wet boundary cells) is pass 2's fallback to
-  // the pass-1 level already written: such cells are left out.
-  const bool pw = k == 1 && !(w > zmx);
-  const unsigned long long m = __ballot(pw);
-  if (m) {
-    const int lane = threadIdx.x & 63;
-    const int leader = __ffsll((long long)m) - 1;
-    unsigned int base = 0;
-    if (lane == leader) base = atomicAdd(W.pw_count, (unsigned int)__popcll(m));
-    base = __shfl(base, leader, 64);
-    if (pw) {
-      const unsigned int below = __builtin_amdgcn_mbcnt_hi(
-          (unsigned int)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned int)m, 0u));
-      W.pw_list[base + below] = (int)i;
-    }
+  recon_store<NT>(W, (int)i, k, w0, gx, gy, k == 1 && !(w > zmx));
+}
+
+// The same over a tile of the stage kernels (swe_tiles.h): the tile's nodes
+// come from its copy, its cells' records (centroid, highest vertex) from the
+// nodes as the setup kernel computes them, and neighbours by local index from
+// LDS, so a cell reads its level, one 16-byte record and its share of the
+// nodes where the other form reads a 32-byte record, vertex and neighbour
+// ids and whole node records, and no gather but the ring's is left.  Bound by
+// HBM: 347 MB of measured traffic at 4M cells (434 before) at 90 % of a
+// copy's rate.  Us per launch, by cells / by tiles: dam break 92.5 / 74.4 (4M
+// cells), 27.9 / 25.5 (1M), 13.5 / 13.6 (250k, bound by the levels' chain), 24
+// ensemble members (0.7M) 20.3 / 18.7.  The vertices are read from LDS twice
+// instead of held (94 to 78 registers, 5 to 6 waves per SIMD: 78.5 to 74.4).
+template <bool HEAD_GRAD, bool NT>
+__global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P, DevState S, DevWork W, int64_t t0,
+                                                           int64_t t1, unsigned long long* r) {
+  extern __shared__ double lds[];
+  __shared__ int s_n;
+  const int64_t tile = t0 + logical_block();
+  const int tid = threadIdx.x;
+  if (r && blockIdx.x == 0 && tid == 0) *r = (unsigned long long)__double_as_longlong(1.0);
+  if (tile >= t1) return;  // padding workgroups of the XCD-aware grid
+  const TileHead h = P.head[tile];
+  const int64_t c0 = tile * kTileCells;
+  const int nc = (int)(M.T - c0 < kTileCells ? M.T - c0 : kTileCells);
+  const int lr = kTileCells + P.sr;
+  // level, centroid, highest vertex (+inf on boundary cells) and centroid
+  // height of own and ring cells; then the list of levels (k_recon1's) in
+  // their place
+  double* const lw = lds;
+  double* const lcx = lw + lr;
+  double* const lcy = lcx + lr;
+  double* const lzm = lcy + lr;
+  double* const lbc = lzm + lr;
+  double* const nx_ = lbc + lr;
+  double* const ny_ = nx_ + P.lo;
+  double* const nz_ = ny_ + P.lo;
+  double* const lvl = lds;                           // [3 kTileCells]
+  int* const lcell = (int*)(lvl + 3 * kTileCells);   // [3 kTileCells]
+  int16_t* const lown = (int16_t*)(lcell + 3 * kTileCells);  // [kTileCells]
+  static_assert(3 * 8 + 3 * 4 + 2 <= 5 * 8, "the list fits the own cells' part of the window");
+  auto lnode = [&](int l) { return V3{nx_[l], ny_[l], nz_[l]}; };
+  const double* const tn = P.tnode + tile * 3 * P.sn;
+  const int* const xl = P.xcell + tile * P.sx;
+  const bool live = tid < nc;
+  const int i = (int)(c0 + (live ? tid : 0));
+  const int xc = tid < P.sr ? xl[tid] : i;
+  const double w = S.w[S.at(i)];
+  const TileCell tc = P.cell[i];
+  V3 nd{0., 0., 0.};
+  if (tid < P.lo) nd = V3{tn[tid], tn[P.sn + tid], tn[2 * P.sn + tid]};
+  if (tid < h.nr) {  // nr <= kTileCells
+    const NRec q = M.nrec[xc];
+    const int l = kTileCells + tid;
+    lw[l] = S.w[S.at(xc)];
+    lcx[l] = q.cx;
+    lcy[l] = q.cy;
+    lzm[l] = q.zmx;
+    lbc[l] = q.bc;
   }
+  if (tid < h.nn0) {
+    nx_[tid] = nd.x;
+    ny_[tid] = nd.y;
+    nz_[tid] = nd.z;
+  }
+  for (int j = tid + kTileCells; j < h.nn0; j += kTileCells) {
+    nx_[j] = tn[j];
+    ny_[j] = tn[P.sn + j];
+    nz_[j] = tn[2 * P.sn + j];
+  }
+  if (tid == 0) s_n = 0;
+  __syncthreads();
+  const uint32_t fl = tc.flags;
+  auto vertex = [&](int k) { return lnode((int)((tc.nodes >> (kLocalBits * k)) & kLocalMask)); };
+  double cx = 0., cy = 0., bc = 0., zmx = 0.;  // zmx: the true highest vertex
+  if (live) {
+    const V3 p0 = vertex(0), p1 = vertex(1), p2 = vertex(2);
+    const V3 c = centroid(p0, p1, p2);
+    cx = c.x;
+    cy = c.y;
+    bc = c.z;
+    zmx = dmax(dmax(p0.z, p1.z), p2.z);
+    lw[tid] = w;
+    lcx[tid] = cx;
+    lcy[tid] = cy;
+    lzm[tid] = (fl & CELL_BND) ? INFINITY : zmx;
+    lbc[tid] = bc;
+  }
+  __syncthreads();
+  const bool on = live && !(M.cinst && !M.bactive[M.cinst[i]]);
+  double wn[3];
+  NRec rn[3];
+  int ln[3];
+#pragma unroll
+  for (int kk = 0; kk < 3; ++kk) {
+    const int l = (int)((tc.nbs >> (kLocalBits * kk)) & kLocalMask);
+    ln[kk] = l >= (int)kLocalMax || !live ? tid : l;  // boundary cells never take the full-wet branch
+    wn[kk] = lw[ln[kk]];
+    rn[kk] = NRec{lcx[ln[kk]], lcy[ln[kk]], lzm[ln[kk]], lbc[ln[kk]]};
+  }
+  int8_t k = 0;
+  if (is_wet(w - bc)) k = !(fl & CELL_BND) && zmx < w ? 2 : 1;
+  const bool own = on && k == 1 && !(w >= zmx);
+  bool nb[3] = {false, false, false}, out[3] = {false, false, false}, any_dry = false;
+  if (on && k == 2) {
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk) {
+      const bool full = rn[kk].zmx < wn[kk], wet = is_wet(wn[kk] - rn[kk].bc);
+      nb[kk] = !full && wet;
+      any_dry = any_dry || (!full && !wet);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk)
+      if (!HEAD_GRAD && nb[kk] && !any_dry) {
+        rn[kk].zmx = wn[kk];
+        out[kk] = ln[kk] >= kTileCells && !(wn[kk] >= M.crec[xl[ln[kk] - kTileCells]].zmax);
+      }
+  }
+  double w0 = w, gx = 0., gy = 0.;
+  if (__syncthreads_or(own || out[0] || out[1] || out[2])) {  // and every read of the window is done
+    int at[3] = {-1, -1, -1};
+    if (own) {
+      at[0] = atomicAdd(&s_n, 1);
+      lcell[at[0]] = i;
+    }
+    lown[tid] = (int16_t)at[0];
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk)
+      if (out[kk]) {
+        at[kk] = atomicAdd(&s_n, 1);
+        lcell[at[kk]] = xl[ln[kk] - kTileCells];
+      }
+    __syncthreads();
+    level_list(M, S, lcell, lvl, s_n);
+    __syncthreads();
+    if (own) w0 = lvl[at[0]];
+#pragma unroll
+    for (int kk = 0; kk < 3; ++kk)
+      if (nb[kk] && !any_dry) {
+        const int q = ln[kk] < kTileCells ? lown[ln[kk]] : at[kk];
+        if (q >= 0) rn[kk].zmx = lvl[q];
+      }
+  }
+  if (!on) return;
+  const V3 p0 = vertex(0), p1 = vertex(1), p2 = vertex(2);  // again, rather than held in registers
+  if (k == 0) {
+    w0 = bc;
+    gradient(p0, p1, p2, gx, gy);
+  } else if (k == 1) {
+    W.wrec1[i] = w0;
+  } else if (!any_dry) {
+    fullwet_plane<HEAD_GRAD>(p0, p1, p2, fl, w, cx, cy, wn, rn, nb, gx, gy);
+  }
+  recon_store<NT>(W, i, k, w0, gx, gy, k == 1 && !(w > zmx));
 }
 
 // ---------------------------------------------------------------- pass 2 --
@@ -1080,8 +1246,19 @@ hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStrea
   return hipGetLastError();
 }
 hipError_t launch_recon1(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
-                         hipStream_t st, bool zero_count, unsigned long long* r) {
+                         hipStream_t st, bool zero_count, unsigned long long* r, const DevTiles* P) {
   if (zero_count) hipLaunchKernelGGL(k_zero_count, dim3(1), dim3(1), 0, st, W.pw_count);
+  if (P) {
+    // the tiles that hold cells of the visited window
+    const int64_t t0 = M.c0 / kTileCells, t1 = (M.c1 + kTileCells - 1) / kTileCells;
+    const dim3 g = grid_for_bs(t1 - t0, 1), b(kTileCells);
+    const unsigned lds = (unsigned)(sizeof(double) * (size_t)(5 * (kTileCells + P->sr) + 3 * P->lo));
+    if ((opts & 1) && M.nt) hipLaunchKernelGGL((k_recon_tile<true, true>), g, b, lds, st, M, *P, S, W, t0, t1, r);
+    else if (opts & 1) hipLaunchKernelGGL((k_recon_tile<true, false>), g, b, lds, st, M, *P, S, W, t0, t1, r);
+    else if (M.nt) hipLaunchKernelGGL((k_recon_tile<false, true>), g, b, lds, st, M, *P, S, W, t0, t1, r);
+    else hipLaunchKernelGGL((k_recon_tile<false, false>), g, b, lds, st, M, *P, S, W, t0, t1, r);
+    return hipGetLastError();
+  }
   const dim3 g = grid_for(M.c1 - M.c0);
   if (opts & 1) {
     if (M.nt) hipLaunchKernelGGL((k_recon1<true, true>), g, dim3(256), 0, st, M, S, W, r);

@@ -237,6 +237,7 @@ struct StageArgs {
   unsigned int* pw_clear = nullptr;
 };
 
+struct DevTiles;
 // the state of cells [0, T) rewritten from S's layout into O's
 hipError_t launch_relayout(const DevState& S, const DevOut& O, int64_t T, hipStream_t st);
 // cells [0, T) between a (T, 3) row-major array (w, u, v per cell) and O's or
@@ -246,9 +247,10 @@ hipError_t launch_rows_out(const DevState& S, double* rows, int64_t T, hipStream
 hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStream_t st);
 // zero_count false: W.pw_count is zero already (the stage before cleared it,
 // or launch_slot_counts); r (may be null): set to 1, for the flux pass that
-// follows
+// follows; P (may be null): by tiles
 hipError_t launch_recon1(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
-                         hipStream_t st, bool zero_count = true, unsigned long long* r = nullptr);
+                         hipStream_t st, bool zero_count = true, unsigned long long* r = nullptr,
+                         const DevTiles* P = nullptr);
 hipError_t launch_zero_count(unsigned int* count, hipStream_t st);
 hipError_t launch_recon2(const DevMesh& M, const DevState& S, const DevWork& W, int opts,
                          hipStream_t st);
@@ -321,7 +323,6 @@ hipError_t launch_adjoint_finish(const DevMesh& M, const DevAdj& J, double* zbar
 // cell's draining step once); this pass's CFL minimum never is.  With
 // from_fluxes the stage's fluxes are already in W (the separate flux pass
 // of a CFL step's first stage) and are read instead of evaluated.
-struct DevTiles;
 // the tiles' data fits the stage kernels' LDS
 bool fused_fits(const DevTiles& P);
 // the tiles' copies of the static geometry, after launch_setup_geometry
