@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -15,7 +16,16 @@
 
 using namespace swe;
 
+// Device memory that a solver's adjoint, tangent and diagnostic calls work in,
+// kept from one call to the next (up to kKeepBytes) until the solver goes.
+struct swe_workspace {
+  char* p = nullptr;
+  size_t bytes = 0;
+  bool busy = false;
+};
+
 struct swe_solver {
+  swe_workspace work;
   int device = 0;
   hipStream_t stream = nullptr;
   int flux = 1, ws = 2, opts = 0;
@@ -89,10 +99,101 @@ int dev_fail(hipError_t e, const char* what) {
   return fail(SWE_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Kept workspaces.  Mapping and unmapping a call's memory cost as much as
+// tens of its small kernels.  Ms per pass, allocated each time / kept:
+// inversion gradient of 250k cells (0.9 GB) 10.3 / 8.9, of a batch of 1.1M
+// (2.7 GB) 36.0 / 34.4, tangent run of 60k cells 1.64 / 1.53.
+// All solvers of a process together keep at most kKeepBytes; a call that needs
+// more allocates and frees its own, and an allocation that fails takes back
+// what idle solvers keep and is tried again.
+constexpr size_t kKeepBytes = size_t(16) << 30;  // a nineteenth of the card
+std::mutex g_work_mutex;
+std::vector<swe_workspace*>& g_work = *new std::vector<swe_workspace*>;  // those that hold memory; outlives every solver
+size_t g_work_bytes = 0;
+
+void work_free(swe_workspace* w) {  // g_work_mutex held, w not busy
+  if (!w->p) return;
+  (void)hipFree(w->p);
+  g_work_bytes -= w->bytes;
+  g_work.erase(std::find(g_work.begin(), g_work.end(), w));
+  w->p = nullptr;
+  w->bytes = 0;
+}
+
+hipError_t dev_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  std::lock_guard<std::mutex> lock(g_work_mutex);
+  bool freed = false;
+  const std::vector<swe_workspace*> held = g_work;
+  for (swe_workspace* w : held)
+    if (!w->busy) {
+      work_free(w);
+      freed = true;
+    }
+  if (!freed) return e;
+  (void)hipGetLastError();  // the failure that is mended here
+  return hipMalloc(p, bytes);
+}
+
+// One call's device memory on a solver: parts of the kept block, or
+// allocations of its own that go with it.  The solver's stream has finished
+// with the memory when this goes.
+class CallMemory {
+ public:
+  // total: the sum of part_bytes() of what will be asked for
+  CallMemory(swe_solver* s, size_t total) : s_(s) {
+    std::lock_guard<std::mutex> lock(g_work_mutex);
+    swe_workspace& w = s->work;
+    if (w.busy) return;  // another thread's call on this solver
+    if (w.bytes < total) {
+      work_free(&w);
+      if (total > kKeepBytes || g_work_bytes + total > kKeepBytes) return;
+      if (hipMalloc((void**)&w.p, total) != hipSuccess) {  // tried part by part below
+        (void)hipGetLastError();
+        w.p = nullptr;
+        return;
+      }
+      w.bytes = total;
+      g_work.push_back(&w);
+      g_work_bytes += total;
+    }
+    w.busy = kept_ = true;
+  }
+  ~CallMemory() {
+    (void)hipStreamSynchronize(s_->stream);  // cleanup: errors are reported where they occur
+    for (void* p : own_) (void)hipFree(p);
+    if (!kept_) return;
+    std::lock_guard<std::mutex> lock(g_work_mutex);
+    s_->work.busy = false;
+  }
+  CallMemory(const CallMemory&) = delete;
+  CallMemory& operator=(const CallMemory&) = delete;
+  static size_t part_bytes(int64_t bytes) { return (size_t(std::max<int64_t>(bytes, 8)) + 255) / 256 * 256; }
+  template <class T>
+  hipError_t part(T** p, int64_t bytes) {
+    const size_t n = part_bytes(bytes);
+    if (kept_ && used_ + n <= s_->work.bytes) {
+      *p = (T*)(s_->work.p + used_);
+      used_ += n;
+      return hipSuccess;
+    }
+    const hipError_t e = dev_malloc((void**)p, n);
+    if (e == hipSuccess) own_.push_back((void*)*p);
+    return e;
+  }
+
+ private:
+  swe_solver* s_;
+  bool kept_ = false;
+  size_t used_ = 0;
+  std::vector<void*> own_;
+};
+
 template <class T>
 hipError_t dalloc(swe_solver* s, T** p, int64_t n) {
   size_t bytes = sizeof(T) * size_t(std::max<int64_t>(n, 1));
-  hipError_t e = hipMalloc((void**)p, bytes);
+  hipError_t e = dev_malloc((void**)p, bytes);
   if (e == hipSuccess) s->allocs.push_back(*p);
   return e;
 }
@@ -497,6 +598,10 @@ void swe_destroy(swe_solver* s) {  // teardown: failures cannot be reported
   if (s->graph) (void)hipGraphExecDestroy(s->graph);
   for (void* p : s->allocs) (void)hipFree(p);
   if (s->dts) (void)hipFree(s->dts);
+  {
+    std::lock_guard<std::mutex> lock(g_work_mutex);
+    work_free(&s->work);
+  }
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -570,8 +675,8 @@ static int edge_and_src(swe_solver* s, double* edg, double* src) {
   if (int rc = set_device(s)) return rc;
   double *de = nullptr, *ds = nullptr;
   size_t n = size_t(6 * std::max<int64_t>(s->E, 1));
-  SWE_CHECK(hipMalloc((void**)&de, sizeof(double) * n), "hipMalloc");
-  hipError_t e = hipMalloc((void**)&ds, sizeof(double) * n);
+  SWE_CHECK(dev_malloc((void**)&de, sizeof(double) * n), "hipMalloc");
+  hipError_t e = dev_malloc((void**)&ds, sizeof(double) * n);
   if (e != hipSuccess) { (void)hipFree(de); return dev_fail(e, "hipMalloc"); }
   e = hipMemsetAsync(de, 0, sizeof(double) * n, s->stream);
   if (e == hipSuccess) e = hipMemsetAsync(ds, 0, sizeof(double) * n, s->stream);
@@ -613,7 +718,7 @@ int swe_get_max_wp(swe_solver* s, double* max_wp) {
   if (!s || !max_wp) return fail(SWE_ERR_ARG, "null argument");
   if (int rc = set_device(s)) return rc;
   double* d = nullptr;
-  SWE_CHECK(hipMalloc((void**)&d, sizeof(double) * size_t(std::max<int64_t>(s->V, 1))), "hipMalloc");
+  SWE_CHECK(dev_malloc((void**)&d, sizeof(double) * size_t(std::max<int64_t>(s->V, 1))), "hipMalloc");
   hipError_t e = launch_max_wp(s->M, s->W, d, s->stream);
   int rc = (e != hipSuccess) ? dev_fail(e, "max_wp") : download(s, max_wp, d, sizeof(double) * size_t(s->V));
   (void)hipStreamSynchronize(s->stream);
@@ -637,7 +742,7 @@ int swe_reconstruct(swe_solver* s, int64_t cell, int kind, double* out5) {
   DevState S = state_of(s, s->cur);
   SWE_CHECK(reconstruct(s, S), "reconstruction");
   double* d = nullptr;
-  SWE_CHECK(hipMalloc((void**)&d, 5 * sizeof(double)), "hipMalloc");
+  SWE_CHECK(dev_malloc((void**)&d, 5 * sizeof(double)), "hipMalloc");
   hipError_t e = launch_reconstruct_one(s->M, S, s->W, int(cell), kind, s->opts, d, s->stream);
   int rc = (e != hipSuccess) ? dev_fail(e, "reconstruct") : download(s, out5, d, 5 * sizeof(double));
   (void)hipStreamSynchronize(s->stream);
@@ -656,7 +761,7 @@ int swe_edge_flux(swe_solver* s, int flux, int wavespeed, int64_t e, int64_t fro
     return fail(SWE_ERR_ARG, "cell index out of range");
   if (int rc = set_device(s)) return rc;
   double* d = nullptr;
-  SWE_CHECK(hipMalloc((void**)&d, 4 * sizeof(double)), "hipMalloc");
+  SWE_CHECK(dev_malloc((void**)&d, 4 * sizeof(double)), "hipMalloc");
   hipError_t he = launch_edge_flux_one(s->M, state_of(s, s->cur), s->W, flux, wavespeed, int(e), int(from),
                                        int(to), s->cor, d, s->stream);
   double o[4] = {0., 0., 0., 0.};
@@ -676,7 +781,7 @@ int swe_rhs(swe_solver* s, int64_t cell, double dt, double* out3) {
   if (int rc = materialize_fluxes(s)) return rc;
   DevState S = state_of(s, s->cur);
   double* d = nullptr;
-  SWE_CHECK(hipMalloc((void**)&d, 3 * sizeof(double)), "hipMalloc");
+  SWE_CHECK(dev_malloc((void**)&d, 3 * sizeof(double)), "hipMalloc");
   hipError_t e = launch_drain(s->M, S, s->W, s->opts, s->stream);
   if (e == hipSuccess) e = launch_rhs_one(s->M, S, s->W, int(cell), dt, s->cor, friction(s), d, s->stream);
   int rc = (e != hipSuccess) ? dev_fail(e, "rhs") : download(s, out3, d, 3 * sizeof(double));
@@ -693,7 +798,7 @@ int swe_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nsteps) {
   if (int rc = set_device(s)) return rc;
   if (nsteps > s->dts_cap) {
     if (s->dts) { (void)hipStreamSynchronize(s->stream); (void)hipFree(s->dts); s->dts = nullptr; }
-    SWE_CHECK(hipMalloc((void**)&s->dts, sizeof(double) * size_t(nsteps)), "hipMalloc");
+    SWE_CHECK(dev_malloc((void**)&s->dts, sizeof(double) * size_t(nsteps)), "hipMalloc");
     s->dts_cap = nsteps;
   }
   for (int64_t k = 0; k < nsteps; ++k)
@@ -1011,7 +1116,7 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
     int nst = scheme == SWE_SCHEME_EULER ? 1 : (scheme == SWE_SCHEME_SSPRK2 ? 2 : 3);
     if (nsteps > s->dts_cap) {
       if (s->dts) { (void)hipStreamSynchronize(s->stream); (void)hipFree(s->dts); s->dts = nullptr; }
-      SWE_CHECK(hipMalloc((void**)&s->dts, sizeof(double) * size_t(nsteps)), "hipMalloc");
+      SWE_CHECK(dev_malloc((void**)&s->dts, sizeof(double) * size_t(nsteps)), "hipMalloc");
       s->dts_cap = nsteps;
     }
     for (int64_t k = 0; k < nsteps && !rc; ++k) {
@@ -1339,17 +1444,17 @@ int swe_integrals(swe_solver* s, double* out3, double* per_cell) {
   DevState S = state_of(s, s->cur);
   SWE_CHECK(reconstruct(s, S), "reconstruction");
   const int64_t nb = integrals_blocks(s->M);
+  const int64_t nd = 8 * (3 * nb + 3), np = per_cell ? 24 * s->T : 0;
   double *d = nullptr, *pc = nullptr;
-  SWE_CHECK(hipMalloc((void**)&d, sizeof(double) * size_t(3 * nb + 3)), "hipMalloc");
+  CallMemory mem(s, CallMemory::part_bytes(nd) + (per_cell ? CallMemory::part_bytes(np) : 0));
+  SWE_CHECK(mem.part(&d, nd), "hipMalloc");
   hipError_t e = hipSuccess;
-  if (per_cell) e = hipMalloc((void**)&pc, sizeof(double) * size_t(3 * std::max<int64_t>(s->T, 1)));
+  if (per_cell) e = mem.part(&pc, np);
   if (e == hipSuccess) e = launch_integrals(s->M, S, s->W, d + 3, pc, d, s->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(out3, d, 3 * sizeof(double), hipMemcpyDeviceToHost, s->stream);
   if (e == hipSuccess && per_cell)
     e = hipMemcpyAsync(per_cell, pc, sizeof(double) * size_t(3 * s->T), hipMemcpyDeviceToHost, s->stream);
   hipError_t e2 = hipStreamSynchronize(s->stream);
-  (void)hipFree(d);
-  if (pc) (void)hipFree(pc);
   if (e == hipSuccess) e = e2;
   if (e != hipSuccess) return dev_fail(e, "integrals");
   return SWE_OK;
@@ -1394,11 +1499,11 @@ int swe_state_stats(swe_solver* s, double* out5) {
   if (int rc = set_device(s)) return rc;
   const int64_t nb = integrals_blocks(s->M);
   double* d = nullptr;
-  SWE_CHECK(hipMalloc((void**)&d, sizeof(double) * size_t(5 * nb + 5)), "hipMalloc");
+  CallMemory mem(s, CallMemory::part_bytes(8 * (5 * nb + 5)));
+  SWE_CHECK(mem.part(&d, 8 * (5 * nb + 5)), "hipMalloc");
   hipError_t e = launch_stats(s->M, state_of(s, s->cur), d + 5, d, s->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(out5, d, 5 * sizeof(double), hipMemcpyDeviceToHost, s->stream);
   hipError_t e2 = hipStreamSynchronize(s->stream);
-  (void)hipFree(d);
   if (e == hipSuccess) e = e2;
   if (e != hipSuccess) return dev_fail(e, "state_stats");
   return SWE_OK;
@@ -1500,16 +1605,6 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
   StageCoef sc[3];
   const int ns = stage_list(scheme, sc);
   const int64_t nck = (nsteps + K - 1) / K;
-  std::vector<void*> mem;
-  auto alloc = [&](auto** p, int64_t bytes) {
-    hipError_t e = hipMalloc((void**)p, size_t(std::max<int64_t>(bytes, 8)));
-    if (e == hipSuccess) mem.push_back((void*)*p);
-    return e;
-  };
-  auto release = [&]() {  // cleanup: errors are reported where they occur
-    (void)hipStreamSynchronize(s->stream);
-    for (void* p : mem) (void)hipFree(p);
-  };
   const int64_t S3 = 3 * T * int64_t(sizeof(double));
   // per-stage work slot: mw, mgx, mgy, wrec1, dtd (T doubles each), f0, f1,
   // f2 (E each), pw_list (T ints), cls (T bytes), pw_count
@@ -1519,20 +1614,25 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
   char* slots = nullptr;
   unsigned int* cnt = nullptr;
   std::vector<unsigned int> hcnt(static_cast<size_t>(K * ns), kPwUnknown);
-  hipError_t e = alloc(&ck, nck * S3);
-  if (e == hipSuccess) e = alloc(&seg, K * S3);
-  if (e == hipSuccess) e = alloc(&stg, K * std::max(ns - 1, 1) * S3);
-  if (e == hipSuccess) e = alloc(&slots, K * ns * slot_bytes);
-  if (e == hipSuccess) e = alloc(&bar_a, S3);
-  if (e == hipSuccess) e = alloc(&bar_b, S3);
-  if (e == hipSuccess) e = alloc(&zb, V * 8);
   // DevAdj work: rb 3T, dtd_own T, dtd_nb 3T, m_cell 3T, sl_edge 6E, drain_h T,
   // w_nb 3T, zc 3T, u0bar 3T, pw_own 4T, pw1_jac 4T, pw_w23bar T, p1bar 3T, zn_acc V,
   // zopp_acc 2E; back 3T and eloc 2E bytes
   const int64_t nwork = 3 * T + T + 3 * T + 3 * T + 6 * E + T + 3 * T + 3 * T + 3 * T + 4 * T + 4 * T + T + 3 * T + V + 2 * E;
-  if (e == hipSuccess) e = alloc(&work, nwork * 8 + ((3 * T + 2 * E + 255) / 256) * 256);
-  if (e == hipSuccess) e = alloc(&cnt, K * ns * int64_t(sizeof(unsigned int)));
-  if (e != hipSuccess) { release(); return dev_fail(e, "hipMalloc (adjoint)"); }
+  const int64_t need[9] = {nck * S3, K * S3, K * std::max(ns - 1, 1) * S3, K * ns * slot_bytes, S3, S3, V * 8,
+                           nwork * 8 + ((3 * T + 2 * E + 255) / 256) * 256, K * ns * int64_t(sizeof(unsigned int))};
+  size_t total = 0;
+  for (int64_t n : need) total += CallMemory::part_bytes(n);
+  CallMemory mem(s, total);
+  hipError_t e = mem.part(&ck, need[0]);
+  if (e == hipSuccess) e = mem.part(&seg, need[1]);
+  if (e == hipSuccess) e = mem.part(&stg, need[2]);
+  if (e == hipSuccess) e = mem.part(&slots, need[3]);
+  if (e == hipSuccess) e = mem.part(&bar_a, need[4]);
+  if (e == hipSuccess) e = mem.part(&bar_b, need[5]);
+  if (e == hipSuccess) e = mem.part(&zb, need[6]);
+  if (e == hipSuccess) e = mem.part(&work, need[7]);
+  if (e == hipSuccess) e = mem.part(&cnt, need[8]);
+  if (e != hipSuccess) return dev_fail(e, "hipMalloc (adjoint)");
   auto slot_work = [&](int64_t idx) {
     char* b = slots + idx * slot_bytes;
     DevWork W{};
@@ -1698,7 +1798,6 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
       s->adj_ms[2] = tm.ms(1, 2) - recompute_ms;
     }
   }
-  release();
   return rc;
 }
 
@@ -1736,7 +1835,8 @@ int swe_tangent_run(swe_solver* s, int scheme, double dt, const double* dts, int
   // intermediates
   const int64_t n8 = 9 * T + V + 5 * T + 3 * E;
   double* buf = nullptr;
-  SWE_CHECK(hipMalloc((void**)&buf, sizeof(double) * size_t(n8)), "hipMalloc (tangent)");
+  CallMemory mem(s, CallMemory::part_bytes(8 * n8));
+  SWE_CHECK(mem.part(&buf, 8 * n8), "hipMalloc (tangent)");
   double* q = buf;
   double* td[3];
   for (int k = 0; k < 3; ++k) { td[k] = q; q += 3 * T; }
@@ -1787,8 +1887,6 @@ int swe_tangent_run(swe_solver* s, int scheme, double dt, const double* dts, int
   } else {
     if (ms) *ms = tm.ms(0, 1);
   }
-  (void)hipStreamSynchronize(s->stream);  // cleanup: errors were reported above
-  (void)hipFree(buf);
   return rc;
 }
 
