@@ -349,8 +349,8 @@ __global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P
   const int nc = (int)(M.T - c0 < kTileCells ? M.T - c0 : kTileCells);
   const int lr = kTileCells + P.sr;
   // level, centroid, highest vertex (+inf on boundary cells) and centroid
-  // height of own and ring cells; then the list of levels (k_recon1's) in
-  // their place
+  // height of own and ring cells; then, in their place, the list of levels:
+  // PartWet1's inputs, the level taking w's place, and each cell's entry
   double* const lw = lds;
   double* const lcx = lw + lr;
   double* const lcy = lcx + lr;
@@ -359,10 +359,11 @@ __global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P
   double* const nx_ = lbc + lr;
   double* const ny_ = nx_ + P.lo;
   double* const nz_ = ny_ + P.lo;
-  double* const lvl = lds;                           // [3 kTileCells]
-  int* const lcell = (int*)(lvl + 3 * kTileCells);   // [3 kTileCells]
-  int16_t* const lown = (int16_t*)(lcell + 3 * kTileCells);  // [kTileCells]
-  static_assert(3 * 8 + 3 * 4 + 2 <= 5 * 8, "the list fits the own cells' part of the window");
+  double* const lvl = lw;
+  double* const vzn = lcx;
+  double* const vzm = lcy;
+  double* const vbc = lzm;
+  int16_t* const lown = (int16_t*)lbc;
   auto lnode = [&](int l) { return V3{nx_[l], ny_[l], nz_[l]}; };
   const double* const tn = P.tnode + tile * 3 * P.sn;
   const int* const xl = P.xcell + tile * P.sx;
@@ -373,10 +374,21 @@ __global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P
   const TileCell tc = P.cell[i];
   V3 nd{0., 0., 0.};
   if (tid < P.lo) nd = V3{tn[tid], tn[P.sn + tid], tn[2 * P.sn + tid]};
+  // the ring cell of this thread, where its level is to be evaluated
+  bool ring = false;
+  double rw = 0., rzn = 0., rzm = 0., rbc = 0.;
   if (tid < h.nr) {  // nr <= kTileCells
     const NRec q = M.nrec[xc];
     const int l = kTileCells + tid;
-    lw[l] = S.w[S.at(xc)];
+    rw = S.w[S.at(xc)];
+    rbc = q.bc;
+    if (!HEAD_GRAD && !(q.zmx < rw) && is_wet(rw - rbc)) {  // partially wet
+      const CellRec f = M.crec[xc];
+      rzn = f.zmin;
+      rzm = f.zmax;
+      ring = !(rw >= rzm);
+    }
+    lw[l] = rw;
     lcx[l] = q.cx;
     lcy[l] = q.cy;
     lzm[l] = q.zmx;
@@ -425,7 +437,7 @@ __global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P
   int8_t k = 0;
   if (is_wet(w - bc)) k = !(fl & CELL_BND) && zmx < w ? 2 : 1;
   const bool own = on && k == 1 && !(w >= zmx);
-  bool nb[3] = {false, false, false}, out[3] = {false, false, false}, any_dry = false;
+  bool nb[3] = {false, false, false}, any_dry = false;
   if (on && k == 2) {
 #pragma unroll
     for (int kk = 0; kk < 3; ++kk) {
@@ -435,33 +447,37 @@ __global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P
     }
 #pragma unroll
     for (int kk = 0; kk < 3; ++kk)
-      if (!HEAD_GRAD && nb[kk] && !any_dry) {
-        rn[kk].zmx = wn[kk];
-        out[kk] = ln[kk] >= kTileCells && !(wn[kk] >= M.crec[xl[ln[kk] - kTileCells]].zmax);
-      }
+      if (nb[kk]) rn[kk].zmx = wn[kk];
   }
   double w0 = w, gx = 0., gy = 0.;
-  if (__syncthreads_or(own || out[0] || out[1] || out[2])) {  // and every read of the window is done
-    int at[3] = {-1, -1, -1};
+  if (__syncthreads_or(own || ring)) {  // and every read of the window is done
+    int at = -1;
     if (own) {
-      at[0] = atomicAdd(&s_n, 1);
-      lcell[at[0]] = i;
+      at = atomicAdd(&s_n, 1);
+      lvl[at] = w;
+      vzn[at] = dmin(dmin(vertex(0).z, vertex(1).z), vertex(2).z);
+      vzm[at] = zmx;
+      vbc[at] = bc;
     }
-    lown[tid] = (int16_t)at[0];
+    lown[tid] = (int16_t)at;
+    int rat = -1;
+    if (ring) {
+      rat = atomicAdd(&s_n, 1);
+      lvl[rat] = rw;
+      vzn[rat] = rzn;
+      vzm[rat] = rzm;
+      vbc[rat] = rbc;
+    }
+    if (tid < h.nr) lown[kTileCells + tid] = (int16_t)rat;
+    __syncthreads();
+    // z0 and z1, z2 enter partwet1_w only through max / min
+    for (int q = tid; q < s_n; q += kTileCells) lvl[q] = partwet1_w(vzn[q], vzn[q], vzm[q], vbc[q], lvl[q]);
+    __syncthreads();
+    if (own) w0 = lvl[at];
 #pragma unroll
     for (int kk = 0; kk < 3; ++kk)
-      if (out[kk]) {
-        at[kk] = atomicAdd(&s_n, 1);
-        lcell[at[kk]] = xl[ln[kk] - kTileCells];
-      }
-    __syncthreads();
-    level_list(M, S, lcell, lvl, s_n);
-    __syncthreads();
-    if (own) w0 = lvl[at[0]];
-#pragma unroll
-    for (int kk = 0; kk < 3; ++kk)
-      if (nb[kk] && !any_dry) {
-        const int q = ln[kk] < kTileCells ? lown[ln[kk]] : at[kk];
+      if (nb[kk]) {
+        const int q = lown[ln[kk]];
         if (q >= 0) rn[kk].zmx = lvl[q];
       }
   }
