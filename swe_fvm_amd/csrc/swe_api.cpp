@@ -47,7 +47,7 @@ struct swe_solver {
   double* sv[3] = {nullptr, nullptr, nullptr};
   int cur = 0;
   DevWork W{};
-  unsigned long long* rbits = nullptr;  // [4]
+  unsigned long long* rbits = nullptr;  // 4 slots of kRSlot words
   int last_r_slot = 3;
   double* dts = nullptr;
   int64_t dts_cap = 0;
@@ -232,7 +232,7 @@ int set_device(swe_solver* s) {
 // flux kernel would have left.
 int materialize_fluxes(swe_solver* s) {
   if (!s->flux_stale) return SWE_OK;
-  SWE_CHECK(launch_flux(s->M, state_of(s, s->stale_in), s->W, s->flux, s->ws, s->cor, s->rbits + s->stale_slot,
+  SWE_CHECK(launch_flux(s->M, state_of(s, s->stale_in), s->W, s->flux, s->ws, s->cor, s->rbits + s->stale_slot * kRSlot,
                         s->flux_items, s->flux_block, s->stream), "flux");
   s->flux_stale = false;
   return SWE_OK;
@@ -267,7 +267,7 @@ int run_stage(swe_solver* s, int in, int u0, int out, double a0, double a1, doub
               double dt_fixed, double cfl, int slot, double* dts_log) {
   DevState S = state_of(s, in);
   const bool fuse = use_fused(s, dt_fixed, slot);
-  SWE_CHECK(reconstruct(s, S, fuse ? nullptr : s->rbits + slot), "reconstruction");
+  SWE_CHECK(reconstruct(s, S, fuse ? nullptr : s->rbits + slot * kRSlot), "reconstruction");
   StageArgs A{a0, a1, coef, dt_fixed, cfl, s->cor, s->rbits, dts_log, friction(s)};
   A.pw_clear = s->W.pw_count;
   if (fuse) {
@@ -277,7 +277,7 @@ int run_stage(swe_solver* s, int in, int u0, int out, double a0, double a1, doub
     s->stale_in = in;
     s->stale_slot = slot;
   } else {
-    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + slot, s->flux_items, s->flux_block, s->stream,
+    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + slot * kRSlot, s->flux_items, s->flux_block, s->stream,
                           kCflTake), "flux");
     s->flux_stale = false;
     if (use_fused_after_flux(s)) {
@@ -440,7 +440,7 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
   ALLOC(s->W.f0, E); ALLOC(s->W.f1, E); ALLOC(s->W.f2, E);
   ALLOC(s->W.dtd, T);
   ALLOC(s->W.pw_list, T); ALLOC(s->W.pw_count, 1);
-  ALLOC(s->rbits, 4);
+  ALLOC(s->rbits, 4 * kRSlot);
   DevGeomOut G{};
   ALLOC(G.cx, T); ALLOC(G.cy, T); ALLOC(G.bc, T);
   ALLOC(G.area, T);
@@ -463,8 +463,8 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
   unsigned long long one;
   double d1 = 1.0;
   std::memcpy(&one, &d1, 8);
-  unsigned long long rinit[4] = {one, one, one, one};
-  if ((e = hipMemcpy(s->rbits, rinit, sizeof(rinit), hipMemcpyHostToDevice)) != hipSuccess)
+  const std::vector<unsigned long long> rinit(size_t(4 * kRSlot), one);
+  if ((e = hipMemcpy(s->rbits, rinit.data(), 8 * rinit.size(), hipMemcpyHostToDevice)) != hipSuccess)
     return bail(e, "hipMemcpy");
   if ((e = hipMemset(s->W.pw_count, 0, sizeof(unsigned int))) != hipSuccess) return bail(e, "hipMemset");
   for (int b = 0; b < 3; ++b) {
@@ -606,6 +606,21 @@ void swe_destroy(swe_solver* s) {  // teardown: failures cannot be reported
   delete s;
 }
 
+static int download(swe_solver* s, void* dst, const void* src, size_t bytes) {
+  SWE_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream), "hipMemcpy");
+  SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
+  return SWE_OK;
+}
+
+// r of a flux pass of a single mesh, the minimum of its lines
+static int download_r(swe_solver* s, int slot, double* r) {
+  unsigned long long bits[kRSlot];
+  if (int rc = download(s, bits, s->rbits + slot * kRSlot, sizeof(bits))) return rc;
+  for (int q = 1; q < kRLines; ++q) bits[0] = std::min(bits[0], bits[q * kRLineWords]);
+  std::memcpy(r, &bits[0], 8);
+  return SWE_OK;
+}
+
 // A state buffer that holds nothing anyone will read: not the current state,
 // not the input of a fused stage whose fluxes are still to be recomputed,
 // and for ensembles not the buffer an Euler step writes next, where finished
@@ -655,19 +670,12 @@ int swe_compute_fluxes(swe_solver* s, double* r) {
   if (int rc = single_mesh(s)) return rc;
   if (int rc = set_device(s)) return rc;
   DevState S = state_of(s, s->cur);
-  SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + 3, s->flux_items, s->flux_block, s->stream), "flux");
+  SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + 3 * kRSlot, s->flux_items, s->flux_block, s->stream), "flux");
   s->flux_stale = false;
   s->last_r_slot = 3;
-  unsigned long long bits;
-  SWE_CHECK(hipMemcpyAsync(&bits, s->rbits + 3, 8, hipMemcpyDeviceToHost, s->stream), "hipMemcpy");
-  SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
-  if (r) std::memcpy(r, &bits, 8);
-  return SWE_OK;
-}
-
-static int download(swe_solver* s, void* dst, const void* src, size_t bytes) {
-  SWE_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream), "hipMemcpy");
-  SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
+  double r3;
+  if (int rc = download_r(s, 3, &r3)) return rc;
+  if (r) *r = r3;
   return SWE_OK;
 }
 
@@ -826,10 +834,8 @@ int swe_cfl_dt(swe_solver* s, double* dt) {
   if (!dt) return fail(SWE_ERR_ARG, "null argument");
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;
-  unsigned long long bits;
-  if (int rc = download(s, &bits, s->rbits + s->last_r_slot, 8)) return rc;
   double r;
-  std::memcpy(&r, &bits, 8);
+  if (int rc = download_r(s, s->last_r_slot, &r)) return rc;
   *dt = 0.15 * r;  // include/TimeDisc.h:13,22
   return SWE_OK;
 }
@@ -839,10 +845,7 @@ int swe_min_len_to_wavespeed(swe_solver* s, double* r) {
   if (!r) return fail(SWE_ERR_ARG, "null argument");
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;
-  unsigned long long bits;
-  if (int rc = download(s, &bits, s->rbits + s->last_r_slot, 8)) return rc;
-  std::memcpy(r, &bits, 8);
-  return SWE_OK;
+  return download_r(s, s->last_r_slot, r);
 }
 
 int64_t swe_num_cells(const swe_solver* s) { return s ? s->T : -1; }
@@ -1142,7 +1145,7 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
         const bool clean = s->pw_clean, fuse = use_fused(s, dt, st);
         s->pw_clean = false;
         timed(0, [&] {
-          return launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, fuse ? nullptr : s->rbits + st,
+          return launch_recon1(s->M, S, s->W, s->opts, s->stream, !clean, fuse ? nullptr : s->rbits + st * kRSlot,
                                tiles_of(s));
         });
         timed(1, [&] { return launch_recon2(s->M, S, s->W, s->opts, s->stream); });
@@ -1156,7 +1159,7 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
           s->stale_slot = st;
         } else {
           timed(2, [&] {
-            return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + st, s->flux_items, s->flux_block,
+            return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + st * kRSlot, s->flux_items, s->flux_block,
                                s->stream, kCflTake);
           });
           s->flux_stale = false;
@@ -1269,7 +1272,7 @@ int swe_autotune(swe_solver* s, int reps, int* flux_items, int* update_items, do
   if (int rc = materialize_fluxes(s)) return rc;  // the free buffer may hold a fused stage's input
   DevState S = state_of(s, s->cur);
   const int scratch = (s->cur + 1) % 3;
-  unsigned long long* rslot = (s->n_inst > 0 ? s->B.rbits : s->rbits) + 3;
+  unsigned long long* rslot = s->n_inst > 0 ? s->B.rbits + 3 : s->rbits + 3 * kRSlot;
   SWE_CHECK(reconstruct(s, S), "reconstruction");
   hipEvent_t e0, e1;
   SWE_CHECK(hipEventCreate(&e0), "hipEventCreate");
@@ -1380,7 +1383,7 @@ int swe_autotune_layout(swe_solver* s, int reps, int* block, double* cost_ms) {
   SWE_CHECK(hipEventCreate(&e1), "hipEventCreate");
   int rc = SWE_OK;
   const bool fused = use_fused(s, 1e-6, 1);
-  unsigned long long* rslot = (s->n_inst > 0 ? s->B.rbits : s->rbits) + 3;
+  unsigned long long* rslot = s->n_inst > 0 ? s->B.rbits + 3 : s->rbits + 3 * kRSlot;
   for (int c = 0; c < kLayoutCandidates && !rc; ++c) {
     rc = swe_set_layout(s, cand[c]);
     if (!rc) rc = swe_autotune(s, reps, &items[c][0], &items[c][1], nullptr);
@@ -1736,7 +1739,7 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
             e = launch_fused(s->M, s->tiles, Sq, Un, O, Wq, A, s->flux, s->ws, s->opts, s->stream, true);
         } else {
           if (e == hipSuccess)  // fixed dt: the CFL reduction is not read
-            e = launch_flux(s->M, Sq, Wq, s->flux, s->ws, s->cor, s->rbits + 3, s->flux_items, s->flux_block, s->stream,
+            e = launch_flux(s->M, Sq, Wq, s->flux, s->ws, s->cor, s->rbits + 3 * kRSlot, s->flux_items, s->flux_block, s->stream,
                             kCflOff);
           if (use_fused_after_flux(s)) {  // draining (stored) and update in one tile kernel
             if (e == hipSuccess)

@@ -36,6 +36,15 @@ __device__ __forceinline__ int logical_block_reversed() {
   int b = blockIdx.x;
   return (b & 7) * per + (per - 1 - (b >> 3));
 }
+// the line of a single mesh's r that this workgroup takes
+__device__ __forceinline__ unsigned long long* r_line(unsigned long long* r) {
+  return r + (blockIdx.x & (kRLines - 1)) * kRLineWords;
+}
+// sets them to 1, by the first kRLines threads of a launch
+__device__ __forceinline__ void reset_r(unsigned long long* r) {
+  if (blockIdx.x == 0 && threadIdx.x < kRLines)
+    r[threadIdx.x * kRLineWords] = (unsigned long long)__double_as_longlong(1.0);
+}
 constexpr int kBlock = 256;  // every launch uses 256-thread workgroups
 __device__ __forceinline__ int64_t global_index() {
   return (int64_t)logical_block() * kBlock + threadIdx.x;
@@ -184,7 +193,15 @@ __device__ __forceinline__ void rhs_compute(const RhsIn& q, double dts, double c
 // the stage's step size: fixed, or cfl times r of the step's first flux pass
 __device__ __forceinline__ double stage_dt(const StageArgs& A) {
   double dt = A.dt_fixed;
-  if (!(dt > 0.)) dt = A.cfl * __longlong_as_double((long long)A.rbits[0]);
+  if (!(dt > 0.)) {
+    unsigned long long b = A.rbits[0];
+#pragma unroll
+    for (int q = 1; q < kRLines; ++q) {  // positive doubles order like their bit patterns
+      const unsigned long long c = A.rbits[q * kRLineWords];
+      b = c < b ? c : b;
+    }
+    dt = A.cfl * __longlong_as_double((long long)b);
+  }
   return dt;
 }
 // an ensemble member's: cfl * r, clipped so that the last step lands on

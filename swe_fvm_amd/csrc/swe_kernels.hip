@@ -249,7 +249,7 @@ __global__ void __launch_bounds__(256) k_recon1(DevMesh M, DevState S, DevWork W
     sh.win.r[tid] = ri;
   }
   if (tid == 0) s_n = 0;
-  if (r && blockIdx.x == 0 && tid == 0) *r = (unsigned long long)__double_as_longlong(1.0);
+  if (r) reset_r(r);
   __syncthreads();
   // finished ensemble members are left alone
   const bool on = live && !(M.cinst && !M.bactive[M.cinst[is]]);
@@ -342,7 +342,7 @@ __global__ void __launch_bounds__(kTileCells) k_recon_tile(DevMesh M, DevTiles P
   __shared__ int s_n;
   const int64_t tile = t0 + logical_block();
   const int tid = threadIdx.x;
-  if (r && blockIdx.x == 0 && tid == 0) *r = (unsigned long long)__double_as_longlong(1.0);
+  if (r) reset_r(r);
   if (tile >= t1) return;  // padding workgroups of the XCD-aware grid
   const TileHead h = P.head[tile];
   const int64_t c0 = tile * kTileCells;
@@ -750,7 +750,7 @@ __global__ void __launch_bounds__(BS) k_flux(DevMesh M, DevState S, DevWork W, d
   }
   if (!CFL) return;
   if (!M.cinst) {
-    block_min_bits(lw, rbits);
+    block_min_bits(lw, r_line(rbits));
     return;
   }
   // ensembles: one r per instance (4 slots apart); a block inside one
@@ -914,9 +914,7 @@ __global__ void __launch_bounds__(BS) k_update(DevMesh M, DevState S, DevState U
   }
 }
 
-__global__ void k_reset_r(unsigned long long* rbits) {
-  *rbits = (unsigned long long)__double_as_longlong(1.0);
-}
+__global__ void k_reset_r(unsigned long long* rbits) { reset_r(rbits); }
 
 // ------------------------------------------------------------ ensembles --
 __global__ void k_batch_reset_r(DevBatch B, int slot) {
@@ -1341,7 +1339,7 @@ hipError_t launch_flux(const DevMesh& M, const DevState& S, const DevWork& W, in
                        double cor, unsigned long long* rbits, int items, int block, hipStream_t st,
                        CflMode mode) {
   const bool cfl = mode != kCflOff || M.cinst;  // ensembles always take their members' minima
-  if (mode == kCflReset && !M.cinst) hipLaunchKernelGGL(k_reset_r, dim3(1), dim3(1), 0, st, rbits);
+  if (mode == kCflReset && !M.cinst) hipLaunchKernelGGL(k_reset_r, dim3(1), dim3(kRLines), 0, st, rbits);
   if (M.e1 <= M.e0) return hipGetLastError();
   if (block != 256 && block != 512) return hipErrorInvalidValue;
   dim3 g = grid_for_bs((M.e1 - M.e0 + items - 1) / items, block), b(block);

@@ -222,13 +222,22 @@ struct DevTan {
   double* dtd;         // [T] draining-dt tangent
 };
 
+// A single mesh keeps the r of a flux pass as kRLines minima on cache lines of
+// their own, one per XCD: every workgroup ends in an atomic minimum, and those
+// of one address go through the memory side one by one, 13 ns each (in
+// the flux pass of 4M cells 11,700 of them, all of its 154 us).  Us per flux
+// pass, one line / eight: 154 / 135 (4M), 16.6 / 12.3 (250k); 1M now 37.1.
+// The readers take the minimum of the lines.  An ensemble's members have an r
+// each, on one line: their workgroups are few.
+constexpr int kRLines = 8, kRLineWords = 16;
+constexpr int kRSlot = kRLines * kRLineWords;  // words of one flux pass's r
 struct StageArgs {
   double a0, a1;       // Shu-Osher weights of U0 and the stage state (a0 = 0: U + RHS)
   double coef;         // stage dt = coef * dt
   double dt_fixed;     // > 0 fixed step, else cfl * r of the step's first flux pass
   double cfl;
   double cor;
-  const unsigned long long* rbits;  // r of the step's first flux pass (double bits)
+  const unsigned long long* rbits;  // r of the step's first flux pass (double bits, kRLines of them)
   double* dts_log;     // receives the step's dt (first stage only), may be null
   double fric;         // linear friction coefficient (0: none)
   double t_end = 0.;   // ensembles: the members' last time
