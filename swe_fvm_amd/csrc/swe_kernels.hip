@@ -586,7 +586,7 @@ __device__ inline void partwet2_muscl(const DevMesh& M, const DevState& S, const
     } else {
       double alpha = 3. * ratio_h;
       double beta = (b13 - b12) / (b13 - b23);
-      double k1 = 1. - bisection(Cubic{0., (alpha - 3.) / beta, (1. + beta - alpha) / (beta * beta)},
+      double k1 = 1. - bisection(DepressedCubic{(alpha - 3.) / beta, (1. + beta - alpha) / (beta * beta)},
                                  0., 1.);
       if (k1 < kTol) {
         fallback = true;
