@@ -47,7 +47,14 @@ __host__ __device__ __forceinline__ int lds_doubles(const DevTiles& P, bool ff, 
 
 __device__ __forceinline__ int local3(uint32_t word, int k) { return (int)((word >> (kLocalBits * k)) & kLocalMask); }
 
-constexpr int kFusedThreads = kTileCells;
+// A launch of no more tiles than the card has CUs leaves a CU one tile, whose
+// ~560 evaluations take a wave per SIMD three rounds one after the other,
+// bound by the latency of its arithmetic: three waves per SIMD take a round
+// each.  Us per fused stage, 256 / 768 threads: 9.6 / 9.0 (1,600 cells), 13.3 /
+// 11.9 (40,000), 11.9 / 11.1 (62,000).  Beyond, a CU has several tiles, which
+// hide each other's latency (and 24 waves would not fit it).  The instance
+// that reads its fluxes has nothing to spread.
+constexpr int kWideThreads = 768, kWideTiles = 256;
 constexpr size_t kTileMaxLds = 64 * 1024;  // of one workgroup
 
 // Gathered per edge from memory, the cells and nodes took 65 gathers of ~26
@@ -65,8 +72,8 @@ constexpr size_t kTileMaxLds = 64 * 1024;  // of one workgroup
 // gathering / staged, dam break: fused stage 283 / 219 (4M cells), 73.3 /
 // 62.1 (1M), 23.1 / 21.5 (250k); after the flux pass 164 / 139, 41.7 / 38.5,
 // 13.7 / 12.6; of 24 ensemble members (0.7M cells) 57.3 / 50.6 and 33.1 / 31.5.
-template <int FLUX, int WS, bool LEN, bool NT, bool FF>
-__global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(DevMesh M, DevTiles P, DevState S, DevState U0,
+template <int FLUX, int WS, bool LEN, bool NT, bool FF, int TH>
+__global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : TH / 256) k_fused(DevMesh M, DevTiles P, DevState S, DevState U0,
                                                       DevOut O, DevWork W, StageArgs A, int64_t t0, int64_t t1,
                                                       int store) {
   extern __shared__ double lds[];
@@ -118,7 +125,8 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
     arear = r[1];
   }
   RhsCell q;
-  q.mu = load_muscl(S, W, i);
+  if (TH > kTileCells && !mine) q.mu = Muscl{0., 0., 0., 0., 0.};
+  else q.mu = load_muscl(S, W, i);
   double w, u, v, w0 = 0., u0 = 0., v0 = 0.;
   w = S.w[S.at(i)];
   u = S.u[S.at(i)];
@@ -133,11 +141,11 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
     // fluxes of the stage's flux pass, written by the separate flux kernel;
     // ne <= kTileMaxEval: at most kFE evaluations per thread, every load of
     // them issued before the first LDS write
-    constexpr int kFE = (kTileMaxEval + kFusedThreads - 1) / kFusedThreads;
+    constexpr int kFE = (kTileMaxEval + TH - 1) / TH;
     int ev[kFE];
 #pragma unroll
     for (int it = 0; it < kFE; ++it) {
-      const int j = tid + it * kFusedThreads;
+      const int j = tid + it * TH;
       ev[it] = j < P.se ? P.evedge[tile * P.se + j] : 0;
     }
     if (ringed) hr = S.w[S.at(xc)] - rbc;
@@ -145,14 +153,14 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
 #pragma unroll
     for (int it = 0; it < kFE; ++it) {
       f0[it] = W.f0[ev[it]];
-      if (tid + it * kFusedThreads < h.na) {
+      if (tid + it * TH < h.na) {
         f1[it] = W.f1[ev[it]];
         f2[it] = W.f2[ev[it]];
       }
     }
 #pragma unroll
     for (int it = 0; it < kFE; ++it) {
-      const int j = tid + it * kFusedThreads;
+      const int j = tid + it * TH;
       if (j < h.ne) sF0[j] = f0[it];
       if (j < h.na) {
         sF1[j] = f1[it];
@@ -175,7 +183,7 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
       if (ringed) hr = S.w[S.at(xc)] - rbc;
       stage_cell(kTileCells + tid, m, xo[2 * tid], xo[2 * tid + 1]);
     }
-    for (int j = tid + kFusedThreads; j < h.nx; j += kFusedThreads)
+    for (int j = tid + TH; j < h.nx; j += TH)
       stage_cell(kTileCells + j, load_muscl(S, W, xl[j]), xo[2 * j], xo[2 * j + 1]);
   }
   if (tid < nn) {
@@ -183,7 +191,7 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
     ny_[tid] = nd.y;
     nz_[tid] = nd.z;
   }
-  for (int j = tid + kFusedThreads; j < nn; j += kFusedThreads) {
+  for (int j = tid + TH; j < nn; j += TH) {
     nx_[j] = tn[j];
     ny_[j] = tn[P.sn + j];
     nz_[j] = tn[2 * P.sn + j];
@@ -207,9 +215,9 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
     // ---- edge fluxes (k_flux's operations), one evaluation per LDS slot;
     // the next evaluation's code is loaded before this one's arithmetic
     auto lmuscl = [&](int l) { return Muscl{cw[l], cgx[l], cgy[l], cu[l], cv[l]}; };
-    for (int j = tid; j < h.ne; j += kFusedThreads) {
+    for (int j = tid; j < h.ne; j += TH) {
       const EvalCode r = rn;
-      if (j + kFusedThreads < h.ne) rn = evl[j + kFusedThreads];
+      if (j + TH < h.ne) rn = evl[j + TH];
       const int f = local3(r.cells, 0), t = local3(r.cells, 1);
       const bool wall = t == (int)kLocalWall;
       const bool all = j < h.na;
@@ -252,7 +260,7 @@ __global__ void __launch_bounds__(kFusedThreads, SWE_FUSED_MIN_WAVES) k_fused(De
       }
     }
     __syncthreads();
-    q.mu = lmuscl(tid);  // read before the draining steps take w0's place
+    q.mu = lmuscl(mine ? tid : 0);  // read before the draining steps take w0's place
   }
 
   // ---- draining time steps of every local cell (k_drain's operations)
@@ -384,26 +392,32 @@ hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, 
   if (!M.cinst && (M.c0 != 0 || M.c1 != M.T)) return hipErrorInvalidValue;
   const int64_t t0 = M.c0 / kTileCells, t1 = (M.c1 + kTileCells - 1) / kTileCells;
   if (t1 <= t0) return hipGetLastError();
-  const dim3 g = grid_for_bs(t1 - t0, 1), b(kFusedThreads);
+  const dim3 g = grid_for_bs(t1 - t0, 1), b(kTileCells);
+  const bool wide = t1 - t0 <= kWideTiles;
   const bool len = (opts & kOptDrainLength) != 0;
   const int sto = store ? 1 : 0;
   const unsigned lds = (unsigned)(sizeof(double) * (size_t)lds_doubles(P, from_fluxes, len));
   if (from_fluxes) {  // the flux scheme does not enter: one instance per drain / store variant
-    if (len && M.nt) hipLaunchKernelGGL((k_fused<0, 0, true, true, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else if (len) hipLaunchKernelGGL((k_fused<0, 0, true, false, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else if (M.nt) hipLaunchKernelGGL((k_fused<0, 0, false, true, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else hipLaunchKernelGGL((k_fused<0, 0, false, false, true>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    if (len && M.nt) hipLaunchKernelGGL((k_fused<0, 0, true, true, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else if (len) hipLaunchKernelGGL((k_fused<0, 0, true, false, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else if (M.nt) hipLaunchKernelGGL((k_fused<0, 0, false, true, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else hipLaunchKernelGGL((k_fused<0, 0, false, false, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
     return hipGetLastError();
   }
-#define SWE_FUSED(F, Wv)                                                                             \
-  if (flux == F && ws == Wv) {                                                                       \
-    if (len && M.nt) hipLaunchKernelGGL((k_fused<F, Wv, true, true, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);   \
-    else if (len) hipLaunchKernelGGL((k_fused<F, Wv, true, false, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);     \
-    else if (M.nt) hipLaunchKernelGGL((k_fused<F, Wv, false, true, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);    \
-    else hipLaunchKernelGGL((k_fused<F, Wv, false, false, false>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);             \
-    return hipGetLastError();                                                                        \
+#define SWE_FUSED_TH(F, Wv, LEN, NT, TH)                                                                              \
+  hipLaunchKernelGGL((k_fused<F, Wv, LEN, NT, false, TH>), g, dim3(TH), lds, st, M, P, S, U0, O, W, A, t0, t1, sto)
+#define SWE_FUSED(F, Wv)                                                                                             \
+  if (flux == F && ws == Wv) {                                                                                       \
+    if (len && M.nt) SWE_FUSED_TH(F, Wv, true, true, kTileCells);                                                    \
+    else if (M.nt) SWE_FUSED_TH(F, Wv, false, true, kTileCells);                                                     \
+    else if (len && wide) SWE_FUSED_TH(F, Wv, true, false, kWideThreads);                                            \
+    else if (wide) SWE_FUSED_TH(F, Wv, false, false, kWideThreads);                                                  \
+    else if (len) SWE_FUSED_TH(F, Wv, true, false, kTileCells);                                                      \
+    else SWE_FUSED_TH(F, Wv, false, false, kTileCells);                                                              \
+    return hipGetLastError();                                                                                        \
   }
   SWE_FUSED(0, 0) SWE_FUSED(0, 1) SWE_FUSED(0, 2) SWE_FUSED(1, 0) SWE_FUSED(1, 1) SWE_FUSED(1, 2)
+#undef SWE_FUSED_TH
 #undef SWE_FUSED
   return hipErrorInvalidValue;
 }

@@ -84,3 +84,17 @@ def test_unusual_coordinates_keep_the_separate_kernels(change):
     sd.run("SSPRK2", 2, dt=dt)
     orc.run("SSPRK2", 2, dt=dt)
     assert np.array_equal(sd.GetVolField(), orc.state(), equal_nan=True)
+
+
+@pytest.mark.parametrize("opts", [0, swe.OPT_DRAIN_LENGTH])
+@pytest.mark.parametrize("nx, ny", [(127, 129), (128, 128), (129, 128)])  # 256 tiles, the last cut short or not; 258
+def test_around_a_tile_per_compute_unit(nx, ny, opts):
+    xyz, topo = swe.StructTriangMesh(nx, ny, 0.02)
+    prim = state(xyz, topo, 5)
+    sd = swe.SpaceDisc(swe.Fluxes.HLLC[swe.Wavespeeds.Einfeldt], swe.Domain(xyz, topo), prim, options=opts)
+    orc = O.OracleSolver(xyz, topo.tables(), "HLLC", "Einfeldt", opts=opts)
+    orc.set_state(prim)
+    for scheme, dt in (("SSPRK2", 0.0), ("Euler", 1e-3)):
+        sd.run(scheme, 2, dt=dt)
+        orc.run(scheme, 2, dt=dt, cfl=0.15)
+        assert np.array_equal(sd.GetVolField(), orc.state()), scheme
