@@ -31,6 +31,7 @@ struct swe_solver {
   int flux = 1, ws = 2, opts = 0;
   int flux_items = 2, upd_items = 1;  // work items per thread (swe_autotune)
   int flux_block = 256, upd_block = 256;  // threads per workgroup (swe_autotune)
+  bool tuned = false;  // they were set: flux_items_of takes them as they are
   double cor = 0., tau = 0.;
   int64_t T = 0, E = 0, V = 0;
   std::vector<void*> allocs;
@@ -225,6 +226,13 @@ int set_device(swe_solver* s) {
   return SWE_OK;
 }
 
+// Edges per thread of the flux pass.  Untuned, two, whose loads overlap; but
+// one while two would leave SIMDs without a wave (64 lanes x 1,024 SIMDs x 2
+// edges): there a second edge only makes the chain longer.  Us per pass, two /
+// one: 6.1 / 4.7 (1,600 cells), 6.8 / 5.3 (5,000), 7.5 / 5.2 (40,000); 12.4 /
+// 12.9 (250k), 36.2 / 38.2 (1M).
+int flux_items_of(const swe_solver* s) { return !s->tuned && s->M.e1 - s->M.e0 < 64 * 1024 * 2 ? 1 : s->flux_items; }
+
 // The fluxes and CFL minimum of the last fused stage, recomputed into W and
 // its r slot from that stage's input (still intact: no stage writes its own
 // input) and its reconstruction, for the getters that read them and before
@@ -233,7 +241,7 @@ int set_device(swe_solver* s) {
 int materialize_fluxes(swe_solver* s) {
   if (!s->flux_stale) return SWE_OK;
   SWE_CHECK(launch_flux(s->M, state_of(s, s->stale_in), s->W, s->flux, s->ws, s->cor, s->rbits + s->stale_slot * kRSlot,
-                        s->flux_items, s->flux_block, s->stream), "flux");
+                        flux_items_of(s), s->flux_block, s->stream), "flux");
   s->flux_stale = false;
   return SWE_OK;
 }
@@ -277,7 +285,7 @@ int run_stage(swe_solver* s, int in, int u0, int out, double a0, double a1, doub
     s->stale_in = in;
     s->stale_slot = slot;
   } else {
-    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + slot * kRSlot, s->flux_items, s->flux_block, s->stream,
+    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + slot * kRSlot, flux_items_of(s), s->flux_block, s->stream,
                           kCflTake), "flux");
     s->flux_stale = false;
     if (use_fused_after_flux(s)) {
@@ -670,7 +678,7 @@ int swe_compute_fluxes(swe_solver* s, double* r) {
   if (int rc = single_mesh(s)) return rc;
   if (int rc = set_device(s)) return rc;
   DevState S = state_of(s, s->cur);
-  SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + 3 * kRSlot, s->flux_items, s->flux_block, s->stream), "flux");
+  SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + 3 * kRSlot, flux_items_of(s), s->flux_block, s->stream), "flux");
   s->flux_stale = false;
   s->last_r_slot = 3;
   double r3;
@@ -891,7 +899,7 @@ static int batch_step(swe_solver* s, int scheme, double cfl, double t_end) {
       continue;
     }
     // slot 0 holds the step's r, set to 1 at the end of the step before
-    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->B.rbits + q, s->flux_items, s->flux_block, s->stream), "flux");
+    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->B.rbits + q, flux_items_of(s), s->flux_block, s->stream), "flux");
     if (use_fused_after_flux(s)) {
       SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->flux, s->ws,
                              s->opts, s->stream, false, true), "fused from fluxes");
@@ -1159,7 +1167,7 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
           s->stale_slot = st;
         } else {
           timed(2, [&] {
-            return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + st * kRSlot, s->flux_items, s->flux_block,
+            return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->rbits + st * kRSlot, flux_items_of(s), s->flux_block,
                                s->stream, kCflTake);
           });
           s->flux_stale = false;
@@ -1220,7 +1228,8 @@ int swe_set_tuning(swe_solver* s, int flux_items, int update_items) {
   if (flux_items != 1 && flux_items != 2 && flux_items != 4)
     return fail(SWE_ERR_ARG, "flux_items must be 1, 2 or 4");
   if (update_items != 1 && update_items != 2) return fail(SWE_ERR_ARG, "update_items must be 1 or 2");
-  if (s->flux_items != flux_items || s->upd_items != update_items) {
+  if (!s->tuned || s->flux_items != flux_items || s->upd_items != update_items) {
+    s->tuned = true;
     s->flux_items = flux_items;
     s->upd_items = update_items;
     if (s->graph) {  // a captured ensemble step holds the old launches
@@ -1396,7 +1405,7 @@ int swe_autotune_layout(swe_solver* s, int reps, int* block, double* cost_ms) {
       hipError_t e = launch_recon1(s->M, S, s->W, s->opts, s->stream, true, nullptr, tiles_of(s));
       if (e == hipSuccess) e = launch_recon2(s->M, S, s->W, s->opts, s->stream);
       if (e == hipSuccess)
-        e = launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, rslot, s->flux_items, s->flux_block, s->stream);
+        e = launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, rslot, flux_items_of(s), s->flux_block, s->stream);
       if (e == hipSuccess && fused)
         e = launch_fused(s->M, s->tiles, S, S, O, s->W, A, s->flux, s->ws, s->opts, s->stream, false, true);
       if (e == hipSuccess && !fused) e = launch_drain(s->M, S, s->W, s->opts, s->stream);
@@ -1739,7 +1748,7 @@ int swe_adjoint_run(swe_solver* s, int scheme, double dt, const double* dts, int
             e = launch_fused(s->M, s->tiles, Sq, Un, O, Wq, A, s->flux, s->ws, s->opts, s->stream, true);
         } else {
           if (e == hipSuccess)  // fixed dt: the CFL reduction is not read
-            e = launch_flux(s->M, Sq, Wq, s->flux, s->ws, s->cor, s->rbits + 3 * kRSlot, s->flux_items, s->flux_block, s->stream,
+            e = launch_flux(s->M, Sq, Wq, s->flux, s->ws, s->cor, s->rbits + 3 * kRSlot, flux_items_of(s), s->flux_block, s->stream,
                             kCflOff);
           if (use_fused_after_flux(s)) {  // draining (stored) and update in one tile kernel
             if (e == hipSuccess)
