@@ -499,24 +499,44 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
     if (plain_geometry(V, px.data(), py.data(), E, ep0.data(), ep1.data()) &&
         build_stage_tables(T, tp.data(), tt.data(), te.data(), flag.data(), et0.data(), et1.data(), ep0.data(),
                            ep1.data(), stt)) {
-      TileHead* dhead;
-      TileCell* dcell;
-      int *dxcell, *dnode, *devedge;
-      RingCode* dxcode;
-      EvalCode* dev;
-      double *dtnode, *dtxc, *dtring;
+      // one block for the tables and the tiles' geometry; the tables of small
+      // meshes cross in one copy (an allocation and a copy for each made a
+      // solver of 1,600 cells 0.15 ms slower to build, one of 40,000 0.4 ms)
       const int64_t nt = stt.ntiles;
-#define UP(dst, v)                                                                                       \
-  if ((e = dalloc(s, &dst, int64_t(v.size()))) != hipSuccess) return bail(e, "hipMalloc");                \
-  if (!v.empty() && (e = hipMemcpy(dst, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice)) != hipSuccess) \
-    return bail(e, "hipMemcpy");
-      UP(dhead, stt.head) UP(dcell, stt.cell) UP(dxcell, stt.xcell) UP(dxcode, stt.xcode) UP(dnode, stt.node)
-      UP(dev, stt.ev) UP(devedge, stt.evedge)
-#undef UP
-#define ALLOC(ptr, n) if ((e = dalloc(s, &ptr, n)) != hipSuccess) return bail(e, "hipMalloc")
-      ALLOC(dtnode, 3 * nt * stt.sn); ALLOC(dtxc, 2 * nt * stt.sx); ALLOC(dtring, 2 * nt * stt.sr);
-#undef ALLOC
-      s->tiles = DevTiles{dhead, dcell, dxcell, dxcode, dnode, dev, devedge, dtnode, dtxc, dtring, nt,
+      size_t end = 0;
+      auto place = [&](size_t bytes) {
+        const size_t at = end;
+        end += (bytes + 255) / 256 * 256;
+        return at;
+      };
+      struct Part {
+        const void* src;
+        size_t bytes, at;
+      };
+      auto table = [&](const auto& v) { return Part{v.data(), sizeof(v[0]) * v.size(), place(sizeof(v[0]) * v.size())}; };
+      const Part part[7] = {table(stt.head), table(stt.cell), table(stt.xcell), table(stt.xcode),
+                            table(stt.node), table(stt.ev),   table(stt.evedge)};
+      const size_t tables = end;
+      const size_t anode = place(sizeof(double) * size_t(3 * nt * stt.sn));
+      const size_t axc = place(sizeof(double) * size_t(2 * nt * stt.sx));
+      const size_t aring = place(sizeof(double) * size_t(2 * nt * stt.sr));
+      char* base = nullptr;
+      if ((e = dalloc(s, &base, int64_t(end))) != hipSuccess) return bail(e, "hipMalloc");
+      if (tables <= (size_t(4) << 20)) {
+        std::vector<char> host(tables);
+        for (const Part& q : part)
+          if (q.bytes) std::memcpy(host.data() + q.at, q.src, q.bytes);
+        if (tables && (e = hipMemcpy(base, host.data(), tables, hipMemcpyHostToDevice)) != hipSuccess)
+          return bail(e, "hipMemcpy");
+      } else {
+        for (const Part& q : part)
+          if (q.bytes && (e = hipMemcpy(base + q.at, q.src, q.bytes, hipMemcpyHostToDevice)) != hipSuccess)
+            return bail(e, "hipMemcpy");
+      }
+      auto in = [&](int q) { return base + part[q].at; };
+      s->tiles = DevTiles{(TileHead*)in(0), (TileCell*)in(1), (int*)in(2), (RingCode*)in(3), (int*)in(4),
+                          (EvalCode*)in(5), (int*)in(6), (double*)(base + anode), (double*)(base + axc),
+                          (double*)(base + aring), nt,
                           stt.sx, stt.sr, stt.sn, stt.se, stt.max_own_nodes, stt.max_own_ev};
       s->fused_ok = fused_fits(s->tiles);
     }
