@@ -68,9 +68,9 @@ def kernel_own_bytes(T, E, V):
     cell-update, which the roofline uses)."""
     nodes = 32.0 * V  # the interleaved node records
     return {
-        # w, 32-byte record, vertex ids + flags, neighbour ids, nodes in;
-        # MUSCL (w0, gx, gy) + class out
-        "recon1": T * (8 + 32 + 16 + 12) + nodes + T * (24 + 1),
+        # w, 16-byte tile record, the tile's copy of its nodes (0.75 of 24
+        # bytes per cell) in; MUSCL (w0, gx, gy) + class out
+        "recon1": T * (8 + 16 + 18) + T * (24 + 1),
         # class of every cell (pass 2 itself is sparse)
         "recon2": T * 1.0,
         # edge ends/cells, CFL length, per-cell MUSCL + class + u, v +
@@ -80,13 +80,14 @@ def kernel_own_bytes(T, E, V):
         "drain": T * (8 + 12 + 12 + 4) + E * 8 + nodes + T * 8,
         # state (+ U0), tp, te, tt, cflag, MUSCL, class, F, dtd, nodes in; state out
         "update": T * (24 + 24 + 36 + 4 + 24 + 1 + 8) + E * 24 + nodes + T * 24,
-        # state (+ U0), vertex ids + flags, tile codes, MUSCL, class,
-        # centroids, edge records, nodes in; state out (fluxes and draining
-        # steps stay in LDS)
-        "fused": T * (24 + 24 + 16 + 12 + 24 + 1 + 16) + E * 16 + nodes + T * 24,
-        # as the fused kernel without the per-edge MUSCL / centroid gathers:
+        # state (+ U0), 16-byte tile record, MUSCL, class, 2.03 evaluation
+        # codes of 8 bytes, the tile's copy of its and the ring's nodes (1.1
+        # of 24 bytes per cell) in; state out (fluxes and draining steps stay
+        # in LDS)
+        "fused": T * (24 + 24 + 16 + 24 + 1 + 16 + 26) + T * 24,
+        # as the fused kernel without the evaluations and the ring's nodes:
         # each edge's flux (24 B) and evaluation index in
-        "fused_ff": T * (24 + 24 + 16 + 12 + 24 + 1) + E * (4 + 24) + nodes + T * 24,
+        "fused_ff": T * (24 + 24 + 16 + 24 + 1 + 18) + E * (4 + 24) + T * 24,
     }
 
 
