@@ -37,14 +37,6 @@ namespace swe {
 #ifndef SWE_FUSED_MIN_WAVES
 #define SWE_FUSED_MIN_WAVES 4
 #endif
-// LDS of a tile, in doubles, the arrays one after the other: the
-// reconstruction of the local cells (w0, gx, gy, u, v, centroid) where the
-// fluxes are evaluated, the nodes (x, y, z), the fluxes.  The draining steps
-// take the place of the cells' w0, which nothing reads after the fluxes.
-__host__ __device__ __forceinline__ int lds_doubles(const DevTiles& P, bool ff, bool len) {
-  return (ff ? kTileCells + P.sr : 7 * (kTileCells + P.sx)) + 3 * (ff && !len ? P.lo : P.sn) + P.se + 2 * P.la;
-}
-
 __device__ __forceinline__ int local3(uint32_t word, int k) { return (int)((word >> (kLocalBits * k)) & kLocalMask); }
 
 // A launch of no more tiles than the card has CUs leaves a CU one tile, whose
@@ -54,8 +46,7 @@ __device__ __forceinline__ int local3(uint32_t word, int k) { return (int)((word
 // 11.9 (40,000), 11.9 / 11.1 (62,000).  Beyond, a CU has several tiles, which
 // hide each other's latency (and 24 waves would not fit it).  The instance
 // that reads its fluxes has nothing to spread.
-constexpr int kWideThreads = 768, kWideTiles = 256;
-constexpr size_t kTileMaxLds = 64 * 1024;  // of one workgroup
+constexpr int kWideThreads = 768, kWideTiles = kCus;
 
 // Gathered per edge from memory, the cells and nodes took 65 gathers of ~26
 // lines per wave (the L1 busy 63 % of the time, its return path 91 %).
@@ -72,7 +63,19 @@ constexpr size_t kTileMaxLds = 64 * 1024;  // of one workgroup
 // gathering / staged, dam break: fused stage 283 / 219 (4M cells), 73.3 /
 // 62.1 (1M), 23.1 / 21.5 (250k); after the flux pass 164 / 139, 41.7 / 38.5,
 // 13.7 / 12.6; of 24 ensemble members (0.7M cells) 57.3 / 50.6 and 33.1 / 31.5.
-template <int FLUX, int WS, bool LEN, bool NT, bool FF, int TH>
+//
+// Those are tiles of Morton-ordered cells.  One that is a strip of a row-ordered
+// mesh has two to three times the cells around it (StructTriangMesh: 130 in
+// the ring and 260 beyond, 56.9 KB, two workgroups to a CU), and one such tile
+// sets the strides of all.  FAR (stage_far) leaves out of LDS what the outer
+// edges of the ring alone need, each once: the cells beyond the ring, gathered
+// from memory by a number that is loaded an evaluation ahead, and the outer
+// nodes, read from the tile's copy (39.2 KB, four workgroups).  Us per fused
+// stage of such a mesh, gathering / staged whole / FAR: 340 / 385 / 288 (4M
+// cells), 83.7 / 100.9 / 79.1 (1M), 35.5 / 40.9 / 34.7 (360,000); with the
+// draining step's edge lengths 357 / 423 / 335, 89.5 / 106.6 / 85.4, 38.2 /
+// 44.0 / 38.0.
+template <int FLUX, int WS, bool LEN, bool NT, bool FF, bool FAR, int TH>
 __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : TH / 256) k_fused(DevMesh M, DevTiles P, DevState S, DevState U0,
                                                       DevOut O, DevWork W, StageArgs A, int64_t t0, int64_t t1,
                                                       int store) {
@@ -86,7 +89,8 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
   const int64_t c0 = tile * kTileCells;
   const int nc = (int)(M.T - c0 < kTileCells ? M.T - c0 : kTileCells);
   const int tid = threadIdx.x;
-  const int lc = kTileCells + P.sx;
+  const int ns = FAR ? P.sr : P.sx;  // of the cells around the tile, those in LDS
+  const int lc = kTileCells + ns;
   double* const cw = lds;  // w0 of the local cells, then the draining steps
   double* const cgx = cw + lc;
   double* const cgy = cgx + lc;
@@ -95,7 +99,7 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
   double* const ccx = cv + lc;
   double* const ccy = ccx + lc;
   double* const sD = lds;
-  const int ln = FF && !LEN ? P.lo : P.sn;
+  const int ln = (FF && !LEN) || FAR ? P.lo : P.sn;
   double* const nx_ = lds + (FF ? kTileCells + P.sr : 7 * lc);
   double* const ny_ = nx_ + ln;
   double* const nz_ = ny_ + ln;
@@ -111,7 +115,7 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
   const bool mine = tid < nc;
   const int i = (int)(c0 + (mine ? tid : 0));
   const bool comb = A.a0 != 0.;
-  const int xc = tid < (FF ? P.sr : P.sx) ? xl[tid] : i;
+  const int xc = tid < (FF ? P.sr : ns) ? xl[tid] : i;
   const TileCell tc = P.cell[i];
   V3 nd{0., 0., 0.};
   if (tid < ln) nd = V3{tn[tid], tn[P.sn + tid], tn[2 * P.sn + tid]};
@@ -136,7 +140,8 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
     u0 = U0.u[U0.at(i)];
     v0 = U0.v[U0.at(i)];
   }
-  const int nn = FF && !LEN ? h.nn0 : h.nn;
+  const int nn = (FF && !LEN) || FAR ? h.nn0 : h.nn;
+  const double* const xo = P.txc + 2 * tile * P.sx;
   if constexpr (FF) {
     // fluxes of the stage's flux pass, written by the separate flux kernel;
     // ne <= kTileMaxEval: at most kFE evaluations per thread, every load of
@@ -177,13 +182,13 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
       ccx[l] = cx;
       ccy[l] = cy;
     };
-    const double* const xo = P.txc + 2 * tile * P.sx;
-    if (tid < h.nx) {
+    const int nx = FAR && h.nx > P.sr ? P.sr : h.nx;
+    if (tid < nx) {
       const Muscl m = load_muscl(S, W, xc);
       if (ringed) hr = S.w[S.at(xc)] - rbc;
       stage_cell(kTileCells + tid, m, xo[2 * tid], xo[2 * tid + 1]);
     }
-    for (int j = tid + TH; j < h.nx; j += TH)
+    for (int j = tid + TH; j < nx; j += TH)
       stage_cell(kTileCells + j, load_muscl(S, W, xl[j]), xo[2 * j], xo[2 * j + 1]);
   }
   if (tid < nn) {
@@ -215,16 +220,47 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
     // ---- edge fluxes (k_flux's operations), one evaluation per LDS slot;
     // the next evaluation's code is loaded before this one's arithmetic
     auto lmuscl = [&](int l) { return Muscl{cw[l], cgx[l], cgy[l], cu[l], cv[l]}; };
+    // FAR: the cell beyond the ring of the next evaluation's edge, by number
+    auto beyond = [&](const EvalCode& r) {
+      const int f = local3(r.cells, 0), t = local3(r.cells, 1);
+      return f >= lc ? f - kTileCells : (t >= lc && t < (int)kLocalMax ? t - kTileCells : -1);
+    };
+    int xn = -1, gn = 0;
+    if (FAR && tid < h.ne && (xn = beyond(rn)) >= 0) gn = xl[xn];
     for (int j = tid; j < h.ne; j += TH) {
       const EvalCode r = rn;
-      if (j + TH < h.ne) rn = evl[j + TH];
+      const int x = xn, gx = gn;
+      if (j + TH < h.ne) {
+        rn = evl[j + TH];
+        if (FAR && (xn = beyond(rn)) >= 0) gn = xl[xn];
+      }
       const int f = local3(r.cells, 0), t = local3(r.cells, 1);
       const bool wall = t == (int)kLocalWall;
       const bool all = j < h.na;
       const int tr = t >= (int)kLocalMax ? f : t;  // boundary edges read their own cell twice: R = L
-      const V3 Pa = lnode(local3(r.nodes, 0)), Pb = lnode(local3(r.nodes, 1));
-      const Muscl mf = lmuscl(f);
-      const double cxf = ccx[f], cyf = ccy[f];
+      auto end = [&](int l) {  // FAR: the nodes that only the ring's outer edges have are not staged
+        return FAR && !all ? V3{tn[l], tn[P.sn + l], tn[2 * P.sn + l]} : lnode(l);
+      };
+      const V3 Pa = end(local3(r.nodes, 0)), Pb = end(local3(r.nodes, 1));
+      Muscl mo{0., 0., 0., 0., 0.};
+      double cxo = 0., cyo = 0.;
+      if (FAR && x >= 0) {
+        mo = load_muscl(S, W, gx);
+        cxo = xo[2 * x];
+        cyo = xo[2 * x + 1];
+      }
+      auto cell = [&](int l, double& cx, double& cy) {
+        if (FAR && l >= lc) {
+          cx = cxo;
+          cy = cyo;
+          return mo;
+        }
+        cx = ccx[l];
+        cy = ccy[l];
+        return lmuscl(l);
+      };
+      double cxf, cyf;
+      const Muscl mf = cell(f, cxf, cyf);
       const V3 E = midpoint(Pa, Pb);
       double le, tx, ty;
       PlainGeometry::edge(Pa, Pb, V3{cxf, cyf, 0.}, le, tx, ty);
@@ -243,11 +279,13 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
         elem_flux(nx, ny, hw, 0., 0., F[0], F[1], F[2]);
       } else {
         const Slot L = slot_value(mf, cxf, cyf, E);
-        const Slot R = slot_value(lmuscl(tr), ccx[tr], ccy[tr], E);
+        double cxt, cyt;
+        const Muscl mt = cell(tr, cxt, cyt);
+        const Slot R = slot_value(mt, cxt, cyt, E);
         if (FLUX == 0) flux_hll<WS>(nx, ny, E.z, L, R, 1.0, A.cor, lw, F, M.eb != 0, all);
         else flux_hllc<WS>(tx, ty, E.z, L, R, 1.0, A.cor, lw, F, M.eb != 0, all);
       }
-      sF0[j] = F[0];
+      sF0[j] = FAR && LEN && !all ? F[0] * le : F[0];
       if (all) {
         sF1[j] = F[1];
         sF2[j] = F[2];
@@ -272,7 +310,7 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
       const int s = local3(slots, k);
       const double fe = sF0[s];
       double out = sgn_pos(fl, k) ? fe : -fe;
-      if (LEN) {
+      if (LEN && (!FAR || s < h.na)) {  // FAR: the outer edges' slots hold the product
         const uint32_t en = evl[s].nodes;
         out = out * edge_len(lnode(local3(en, 0)), lnode(local3(en, 1)));
       }
@@ -379,8 +417,7 @@ hipError_t launch_setup_tiles(const DevMesh& M, const DevTiles& P, hipStream_t s
 }
 
 bool fused_fits(const DevTiles& P) {
-  return sizeof(double) * (size_t)lds_doubles(P, false, true) <= kTileMaxLds &&
-         sizeof(double) * (size_t)lds_doubles(P, true, true) <= kTileMaxLds;
+  return stage_lds(P, false, true, true) <= kTileMaxLds && stage_lds(P, true, false, true) <= kTileMaxLds;
 }
 
 hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, const DevState& U0,
@@ -393,27 +430,32 @@ hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, 
   const int64_t t0 = M.c0 / kTileCells, t1 = (M.c1 + kTileCells - 1) / kTileCells;
   if (t1 <= t0) return hipGetLastError();
   const dim3 g = grid_for_bs(t1 - t0, 1), b(kTileCells);
-  const bool wide = t1 - t0 <= kWideTiles;
+  const bool wide = !M.nt && t1 - t0 <= kWideTiles;
   const bool len = (opts & kOptDrainLength) != 0;
   const int sto = store ? 1 : 0;
-  const unsigned lds = (unsigned)(sizeof(double) * (size_t)lds_doubles(P, from_fluxes, len));
+  const bool far = !from_fluxes && stage_far(P, len, t1 - t0);
+  const unsigned lds = (unsigned)stage_lds(P, from_fluxes, far, len);
   if (from_fluxes) {  // the flux scheme does not enter: one instance per drain / store variant
-    if (len && M.nt) hipLaunchKernelGGL((k_fused<0, 0, true, true, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else if (len) hipLaunchKernelGGL((k_fused<0, 0, true, false, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else if (M.nt) hipLaunchKernelGGL((k_fused<0, 0, false, true, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
-    else hipLaunchKernelGGL((k_fused<0, 0, false, false, true, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    if (len && M.nt) hipLaunchKernelGGL((k_fused<0, 0, true, true, true, false, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else if (len) hipLaunchKernelGGL((k_fused<0, 0, true, false, true, false, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else if (M.nt) hipLaunchKernelGGL((k_fused<0, 0, false, true, true, false, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
+    else hipLaunchKernelGGL((k_fused<0, 0, false, false, true, false, kTileCells>), g, b, lds, st, M, P, S, U0, O, W, A, t0, t1, sto);
     return hipGetLastError();
   }
-#define SWE_FUSED_TH(F, Wv, LEN, NT, TH)                                                                              \
-  hipLaunchKernelGGL((k_fused<F, Wv, LEN, NT, false, TH>), g, dim3(TH), lds, st, M, P, S, U0, O, W, A, t0, t1, sto)
+#define SWE_FUSED_TH(F, Wv, LEN, NT, FAR, TH)                                                                         \
+  hipLaunchKernelGGL((k_fused<F, Wv, LEN, NT, false, FAR, TH>), g, dim3(TH), lds, st, M, P, S, U0, O, W, A, t0, t1, sto)
 #define SWE_FUSED(F, Wv)                                                                                             \
   if (flux == F && ws == Wv) {                                                                                       \
-    if (len && M.nt) SWE_FUSED_TH(F, Wv, true, true, kTileCells);                                                    \
-    else if (M.nt) SWE_FUSED_TH(F, Wv, false, true, kTileCells);                                                     \
-    else if (len && wide) SWE_FUSED_TH(F, Wv, true, false, kWideThreads);                                            \
-    else if (wide) SWE_FUSED_TH(F, Wv, false, false, kWideThreads);                                                  \
-    else if (len) SWE_FUSED_TH(F, Wv, true, false, kTileCells);                                                      \
-    else SWE_FUSED_TH(F, Wv, false, false, kTileCells);                                                              \
+    if (far && len && M.nt) SWE_FUSED_TH(F, Wv, true, true, true, kTileCells);                                       \
+    else if (far && M.nt) SWE_FUSED_TH(F, Wv, false, true, true, kTileCells);                                        \
+    else if (far && len) SWE_FUSED_TH(F, Wv, true, false, true, kTileCells);                                         \
+    else if (far) SWE_FUSED_TH(F, Wv, false, false, true, kTileCells);                                               \
+    else if (len && M.nt) SWE_FUSED_TH(F, Wv, true, true, false, kTileCells);                                        \
+    else if (M.nt) SWE_FUSED_TH(F, Wv, false, true, false, kTileCells);                                              \
+    else if (len && wide) SWE_FUSED_TH(F, Wv, true, false, false, kWideThreads);                                     \
+    else if (wide) SWE_FUSED_TH(F, Wv, false, false, false, kWideThreads);                                           \
+    else if (len) SWE_FUSED_TH(F, Wv, true, false, false, kTileCells);                                               \
+    else SWE_FUSED_TH(F, Wv, false, false, false, kTileCells);                                                       \
     return hipGetLastError();                                                                                        \
   }
   SWE_FUSED(0, 0) SWE_FUSED(0, 1) SWE_FUSED(0, 2) SWE_FUSED(1, 0) SWE_FUSED(1, 1) SWE_FUSED(1, 2)

@@ -2,6 +2,7 @@
 // tables (swe_tiles.cpp) and their device view (swe_fused.hip).
 #pragma once
 
+#include <stddef.h>
 #include <stdint.h>
 
 #include <vector>
@@ -11,7 +12,7 @@ namespace swe {
 #ifndef SWE_TILE_CELLS
 #define SWE_TILE_CELLS 256
 #endif
-constexpr int kTileCells = SWE_TILE_CELLS;      // cells per tile (a build-time knob: 256 or 512)
+constexpr int kTileCells = SWE_TILE_CELLS;      // cells per tile (the tables also build at 512; the stage kernels' local indices hold 256)
 constexpr int kTileMaxLocal = 2 * kTileCells;  // tile cells + ring
 constexpr int kTileMaxEval = 3 * kTileCells;   // edge evaluations per tile (LDS flux slots)
 static_assert(kTileCells == 256 || kTileCells == 512, "tile size");
@@ -116,5 +117,32 @@ struct DevTiles {
   int sx, sr, sn, se;  // strides
   int lo, la;          // the most nodes of a tile's own cells, evaluations of its cells' edges
 };
+
+constexpr size_t kTileMaxLds = 64 * 1024;  // of one workgroup
+constexpr size_t kCuLds = 160 * 1024;
+constexpr int kCus = 256;
+
+// Bytes of LDS of a stage kernel's tile, arrays of doubles one after the
+// other: the reconstruction of the local cells (w0, gx, gy, u, v, centroid)
+// where the fluxes are evaluated (far: without the cells beyond the ring), the
+// nodes (x, y, z; those of the own cells alone where that will do), the
+// fluxes.  The draining steps take the place of the cells' w0, which nothing
+// reads after the fluxes.  ff: the fluxes are read, not evaluated; len:
+// SWE_OPT_DRAIN_LENGTH.
+inline size_t stage_lds(const DevTiles& P, bool ff, bool far, bool len) {
+  const int cells = ff ? kTileCells + P.sr : 7 * (kTileCells + (far ? P.sr : P.sx));
+  const int nodes = (ff && !len) || far ? P.lo : P.sn;
+  return sizeof(double) * size_t(cells + 3 * nodes + P.se + 2 * P.la);
+}
+// Whether a launch of n tiles leaves the cells beyond the ring out of LDS:
+// where all of them would not fit, or leave a CU two workgroups and there are
+// more tiles than that.  At three to a CU the two forms are alike (4M cells,
+// us per fused stage staged whole / far: 272 / 268, 311 / 305; with edge
+// lengths 301 / 312, 350 / 360), at two far is the faster one (335 / 265), but
+// not while all tiles are on the chip at once (307 of them: 17.3 / 18.7).
+inline bool stage_far(const DevTiles& P, bool len, int64_t n) {
+  const size_t whole = stage_lds(P, false, false, len);
+  return whole > kTileMaxLds || (3 * whole > kCuLds && n > 2 * kCus);
+}
 
 }  // namespace swe
