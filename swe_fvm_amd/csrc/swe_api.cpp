@@ -912,22 +912,24 @@ static int batch_step(swe_solver* s, int scheme, double cfl, double t_end) {
     A.t_end = t_end;
     A.pw_clear = s->W.pw_count;
     SWE_CHECK(reconstruct(s, S), "reconstruction");
-    s->pw_clean = true;  // by this stage's last kernel
     if (q > 0 && use_fused(s, 0., q)) {  // the members' step sizes are known: one fused kernel
       SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->flux, s->ws,
                              s->opts, s->stream), "fused");
-      continue;
+    } else {
+      // slot 0 holds the step's r, set to 1 at the end of the step before
+      SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->B.rbits + q, flux_items_of(s), s->flux_block, s->stream), "flux");
+      if (use_fused_after_flux(s)) {
+        SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->flux, s->ws,
+                               s->opts, s->stream, false, true), "fused from fluxes");
+      } else {
+        SWE_CHECK(launch_drain(s->M, S, s->W, s->opts, s->stream), "drain");
+        SWE_CHECK(launch_update(s->M, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->upd_items, s->upd_block, s->stream),
+                  "update");
+      }
     }
-    // slot 0 holds the step's r, set to 1 at the end of the step before
-    SWE_CHECK(launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, s->B.rbits + q, flux_items_of(s), s->flux_block, s->stream), "flux");
-    if (use_fused_after_flux(s)) {
-      SWE_CHECK(launch_fused(s->M, s->tiles, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->flux, s->ws,
-                             s->opts, s->stream, false, true), "fused from fluxes");
-      continue;
-    }
-    SWE_CHECK(launch_drain(s->M, S, s->W, s->opts, s->stream), "drain");
-    SWE_CHECK(launch_update(s->M, S, state_of(s, st[q].u0), out_of(s, st[q].out), s->W, A, s->upd_items, s->upd_block, s->stream),
-              "update");
+    // the stage's last kernel clears the list; where it was not launched the
+    // next user does, or pass 1 would append past the list's end
+    s->pw_clean = true;
   }
   SWE_CHECK(launch_batch_advance(s->B, cfl, t_end, s->stream), "batch_advance");
   if (scheme == SWE_SCHEME_EULER) s->cur = b;

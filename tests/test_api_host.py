@@ -1,0 +1,37 @@
+"""The library's host code over a device that is host memory
+(tests/cpp/api_on_host.cpp): what it does where a launch fails, where threads
+meet, and over sequences of calls."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIP = "/opt/rocm/include"
+EULER, SSPRK2, SSPRK3 = 0, 1, 2
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    if not os.path.exists(os.path.join(HIP, "hip", "hip_runtime.h")):
+        pytest.skip("no HIP headers")
+    out = str(tmp_path_factory.mktemp("api") / "libapi_on_host.so")
+    src = os.path.join(ROOT, "swe_fvm_amd", "csrc")
+    res = subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-shared", "-fPIC", "-pthread", "-D__HIP_PLATFORM_AMD__",
+                          "-Wl,-z,lazy", "-Wl,-Bsymbolic", "-I", HIP, os.path.join(ROOT, "tests", "cpp", "api_on_host.cpp"),
+                          os.path.join(src, "swe_mesh.cpp"), os.path.join(src, "swe_tiles.cpp"), "-o", out],
+                         capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
+    return ctypes.CDLL(out, mode=os.RTLD_LAZY | os.RTLD_LOCAL)
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("scheme, fused, launch", [(EULER, 1, "flux"), (EULER, 1, "fused"), (SSPRK2, 1, "fused"),
+                                                   (SSPRK2, 0, "flux"), (SSPRK3, 0, "drain"), (SSPRK2, 0, "update"),
+                                                   (SSPRK2, 1, "recon1"), (SSPRK2, 1, "recon2")])
+def test_a_failed_launch_leaves_no_longer_list(lib, scheme, fused, launch, graph):
+    lib.list_after_failed_launch.restype = ctypes.c_int64
+    cells = ctypes.c_int64()
+    longest = lib.list_after_failed_launch(launch.encode(), scheme, fused, graph, ctypes.byref(cells))
+    assert cells.value == 192 and longest == cells.value
