@@ -649,6 +649,9 @@ static int download_r(swe_solver* s, int slot, double* r) {
   return SWE_OK;
 }
 
+// the buffer an ensemble's Euler step writes, and returns from
+static int euler_other(const swe_solver* s) { return s->cur == 0 ? 1 : 0; }
+
 // A state buffer that holds nothing anyone will read: not the current state,
 // not the input of a fused stage whose fluxes are still to be recomputed,
 // and for ensembles not the buffer an Euler step writes next, where finished
@@ -656,7 +659,7 @@ static int download_r(swe_solver* s, int slot, double* r) {
 static int free_buffer(const swe_solver* s) {
   for (int b = 0; b < 3; ++b) {
     if (b == s->cur || (s->flux_stale && b == s->stale_in)) continue;
-    if (s->n_inst > 0 && b == (s->cur == 0 ? 1 : 0)) continue;
+    if (s->n_inst > 0 && b == euler_other(s)) continue;
     return b;
   }
   return -1;  // not reached: at most two of the three are taken
@@ -893,7 +896,7 @@ static int batch_step(swe_solver* s, int scheme, double cfl, double t_end) {
   // Euler ping-pongs between two buffers so that a two-step graph returns
   // the state to the buffer it started from
   const int a = s->cur;
-  const int b = (scheme == SWE_SCHEME_EULER) ? (a == 0 ? 1 : 0) : (a + 1) % 3;
+  const int b = (scheme == SWE_SCHEME_EULER) ? euler_other(s) : (a + 1) % 3;
   const int c = (a + 2) % 3;
   struct St { int in, u0, out; double a0, a1, coef; };
   St st[3];
@@ -971,7 +974,7 @@ static int batch_window(swe_solver* s, const std::vector<int>& act, bool euler) 
     s->M.e1 = s->edge_off[size_t(k1) + 1];
   }
   if (!euler) return SWE_OK;
-  const int a = s->cur, b = a == 0 ? 1 : 0;
+  const int a = s->cur, b = euler_other(s);
   auto copy = [&](int64_t c0, int64_t c1) -> int {
     if (c1 <= c0) return SWE_OK;
     if (s->lay_b != 0) {
@@ -1373,7 +1376,9 @@ int swe_set_layout(swe_solver* s, int block) {
   if (int rc = set_device(s)) return rc;
   if (int rc = materialize_fluxes(s)) return rc;  // it reads the stale stage input in the old layout
   const DevState src = state_of(s, s->cur);
-  const int to = (s->cur + 1) % 3;
+  // an ensemble's state stays in the two buffers its Euler steps alternate
+  // between, or a captured pair of steps would not end where it began
+  const int to = s->n_inst > 0 ? euler_other(s) : (s->cur + 1) % 3;
   s->lay_b = block;
   layout_ptrs(s);
   SWE_CHECK(launch_relayout(src, out_of(s, to), s->T, s->stream), "relayout");

@@ -227,3 +227,22 @@ extern "C" int64_t list_after_failed_launch(const char* launch, int scheme, int 
   swe_destroy(s);
   return rc == SWE_OK && failed == SWE_ERR_DEVICE ? fake::list_max : -1;
 }
+
+// Euler steps of an ensemble after `layouts` changes of the state layout:
+// every step adds 1 to w.  Returns the steps that the state shows, or -1.
+extern "C" int64_t euler_steps_after_layouts(int layouts, int graph, int runs, int64_t steps) {
+  Mesh m(4);
+  swe_solver* s = ensemble(m, 3);
+  if (!s) return -1;
+  std::vector<double> prim(size_t(3 * s->T), 0.);
+  int rc = swe_set_state(s, prim.data());
+  for (int k = 0; k < layouts; ++k) rc |= swe_set_layout(s, k % 2 == 0 ? 64 : 0);
+  int64_t done, act;
+  for (int k = 0; k < runs; ++k) rc |= swe_batch_run(s, SWE_SCHEME_EULER, 0.15, 1e9, steps, graph, &done, &act);
+  rc |= swe_get_state(s, prim.data());
+  const int64_t T = s->T;
+  swe_destroy(s);
+  for (int64_t i = 0; i < T; ++i)
+    if (prim[size_t(3 * i)] != prim[0]) rc = SWE_ERR_ARG;
+  return rc == SWE_OK ? int64_t(prim[0]) : -1;
+}

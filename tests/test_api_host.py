@@ -35,3 +35,11 @@ def test_a_failed_launch_leaves_no_longer_list(lib, scheme, fused, launch, graph
     cells = ctypes.c_int64()
     longest = lib.list_after_failed_launch(launch.encode(), scheme, fused, graph, ctypes.byref(cells))
     assert cells.value == 192 and longest == cells.value
+
+
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("layouts", range(5))
+def test_euler_ensembles_after_layout_changes(lib, layouts, graph):
+    lib.euler_steps_after_layouts.restype = ctypes.c_int64
+    for runs, steps in ((1, 6), (2, 3), (1, 67)):
+        assert lib.euler_steps_after_layouts(layouts, graph, runs, ctypes.c_int64(steps)) == runs * steps
