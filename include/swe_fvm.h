@@ -160,6 +160,13 @@ int swe_create(const swe_topology* topo, const double* xyz, int flux, int wavesp
                double tau, int options, int device, swe_solver** out);
 void swe_destroy(swe_solver* s);
 
+/* Gives the device memory that solvers keep for their next swe_adjoint_run,
+ * swe_tangent_run, swe_integrals or swe_state_stats (at most 16 GiB over all
+ * solvers of the process) back to the device, for another allocator to use.
+ * Solvers in such a call keep theirs.  An allocation of this library that
+ * fails does the same by itself. */
+int swe_release_workspaces(void);
+
 /* VolumeField write / read (include/ValueField.h:33-44): primitive (w, u, v),
  * T x 3 host arrays.  Writes store the values as given (no assigner). */
 int swe_set_state(swe_solver* s, const double* prim);

@@ -8,12 +8,12 @@ from .core import (DomainError, DeviceError, Domain, Fluxer, Fluxes, SolverError
                    Solvers, StructTriangMesh, TimeDisc, Topology, Wavespeeds, jittered_mesh,
                    read_msh, OPT_HEAD_GRADIENT, OPT_HEAD_PARTWET2, OPT_FRICTION, OPT_DRAIN_LENGTH,
                    OPT_EXACT_BALANCE, SOLID_WALL, FREE_FLOW, PERIODIC, periodic_pairs, stack_domains,
-                   morton_order, reorder_cells)
+                   morton_order, release_workspaces, reorder_cells)
 
 __all__ = [
     "DomainError", "DeviceError", "Domain", "Fluxer", "Fluxes", "SolverError", "SpaceDisc",
     "Solvers", "StructTriangMesh", "TimeDisc", "Topology", "Wavespeeds", "jittered_mesh",
     "read_msh", "OPT_HEAD_GRADIENT", "OPT_HEAD_PARTWET2", "OPT_FRICTION", "OPT_DRAIN_LENGTH",
     "OPT_EXACT_BALANCE", "SOLID_WALL", "FREE_FLOW", "PERIODIC", "periodic_pairs", "stack_domains",
-    "morton_order", "reorder_cells",
+    "morton_order", "release_workspaces", "reorder_cells",
 ]

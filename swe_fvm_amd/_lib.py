@@ -36,6 +36,7 @@ SIGNATURES = [
     ("swe_mesh_jittered", _int, [_i64, _d, _u64, _d, _d, _d, _pp, _pi64, _pp]),
     ("swe_create", _int, [_p, _p, _int, _int, _d, _d, _int, _int, _pp]),
     ("swe_destroy", None, [_p]),
+    ("swe_release_workspaces", _int, []),
     ("swe_set_state", _int, [_p, _p]),
     ("swe_get_state", _int, [_p, _p]),
     ("swe_compute_interface_values", _int, [_p]),

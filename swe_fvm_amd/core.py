@@ -644,6 +644,12 @@ class SpaceDisc:
 LAYOUTS = (0, 64, 8, 1)  # the candidates of swe_autotune_layout, in its order
 
 
+def release_workspaces():
+    """Gives the device memory that solvers keep between their adjoint, tangent
+    and diagnostic calls back to the device (swe_release_workspaces)."""
+    _check(_lib.load().swe_release_workspaces())
+
+
 def _layout(h):
     b = ctypes.c_int()
     _check(_lib.load().swe_get_layout(h, ctypes.byref(b)))

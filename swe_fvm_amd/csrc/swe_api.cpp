@@ -17,11 +17,13 @@
 using namespace swe;
 
 // Device memory that a solver's adjoint, tangent and diagnostic calls work in,
-// kept from one call to the next (up to kKeepBytes) until the solver goes.
+// kept from one call to the next (up to kKeepBytes) until the solver goes or
+// swe_release_workspaces is called.
 struct swe_workspace {
   char* p = nullptr;
   size_t bytes = 0;
   bool busy = false;
+  swe_workspace *prev = nullptr, *next = nullptr;  // in the list of those that hold memory
 };
 
 struct swe_solver {
@@ -106,33 +108,46 @@ int dev_fail(hipError_t e, const char* what) {
 // (2.7 GB) 36.0 / 34.4, tangent run of 60k cells 1.64 / 1.53.
 // All solvers of a process together keep at most kKeepBytes; a call that needs
 // more allocates and frees its own, and an allocation that fails takes back
-// what idle solvers keep and is tried again.
+// what idle solvers keep and is tried again.  The mutex guards the list and
+// the sum alone: no device call is made under it (hipFree waits for the whole
+// device), so solvers on other threads do not wait for each other.
 constexpr size_t kKeepBytes = size_t(16) << 30;  // a nineteenth of the card
 std::mutex g_work_mutex;
-std::vector<swe_workspace*>& g_work = *new std::vector<swe_workspace*>;  // those that hold memory; outlives every solver
-size_t g_work_bytes = 0;
+swe_workspace* g_work = nullptr;  // those that hold memory
+size_t g_work_bytes = 0;          // theirs, and what is being allocated for one
 
-void work_free(swe_workspace* w) {  // g_work_mutex held, w not busy
-  if (!w->p) return;
-  (void)hipFree(w->p);
+// g_work_mutex held: w's memory, which the caller frees after it
+char* work_take(swe_workspace* w) {
+  char* const p = w->p;
+  if (!p) return nullptr;
   g_work_bytes -= w->bytes;
-  g_work.erase(std::find(g_work.begin(), g_work.end(), w));
+  if (w->next) w->next->prev = w->prev;
+  (w->prev ? w->prev->next : g_work) = w->next;
+  w->prev = w->next = nullptr;
   w->p = nullptr;
   w->bytes = 0;
+  return p;
+}
+// gives back what idle solvers keep; whether there was any
+bool work_release() {
+  for (bool any = false;; any = true) {
+    char* p = nullptr;
+    {
+      std::lock_guard<std::mutex> lock(g_work_mutex);
+      for (swe_workspace* w = g_work; w && !p; w = w->next)
+        if (!w->busy) {
+          p = work_take(w);
+          break;
+        }
+    }
+    if (!p) return any;
+    (void)hipFree(p);
+  }
 }
 
 hipError_t dev_malloc(void** p, size_t bytes) {
-  hipError_t e = hipMalloc(p, bytes);
-  if (e != hipErrorOutOfMemory) return e;
-  std::lock_guard<std::mutex> lock(g_work_mutex);
-  bool freed = false;
-  const std::vector<swe_workspace*> held = g_work;
-  for (swe_workspace* w : held)
-    if (!w->busy) {
-      work_free(w);
-      freed = true;
-    }
-  if (!freed) return e;
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory || !work_release()) return e;
   (void)hipGetLastError();  // the failure that is mended here
   return hipMalloc(p, bytes);
 }
@@ -144,22 +159,32 @@ class CallMemory {
  public:
   // total: the sum of part_bytes() of what will be asked for
   CallMemory(swe_solver* s, size_t total) : s_(s) {
-    std::lock_guard<std::mutex> lock(g_work_mutex);
     swe_workspace& w = s->work;
-    if (w.busy) return;  // another thread's call on this solver
-    if (w.bytes < total) {
-      work_free(&w);
-      if (total > kKeepBytes || g_work_bytes + total > kKeepBytes) return;
-      if (hipMalloc((void**)&w.p, total) != hipSuccess) {  // tried part by part below
-        (void)hipGetLastError();
-        w.p = nullptr;
-        return;
-      }
-      w.bytes = total;
-      g_work.push_back(&w);
-      g_work_bytes += total;
+    char *old = nullptr, *p = nullptr;
+    bool room;
+    {
+      std::lock_guard<std::mutex> lock(g_work_mutex);
+      if (w.busy) return;  // another thread's call on this solver
+      w.busy = true;
+      if ((kept_ = w.bytes >= total)) return;
+      old = work_take(&w);
+      room = total <= kKeepBytes && g_work_bytes <= kKeepBytes - total;
+      if (room) g_work_bytes += total;
     }
-    w.busy = kept_ = true;
+    if (old) (void)hipFree(old);
+    if (room && hipMalloc((void**)&p, total) != hipSuccess) {  // tried part by part below
+      (void)hipGetLastError();
+      p = nullptr;
+    }
+    std::lock_guard<std::mutex> lock(g_work_mutex);
+    kept_ = w.busy = p != nullptr;
+    if (!p && room) g_work_bytes -= total;
+    if (!p) return;
+    w.p = p;
+    w.bytes = total;
+    w.next = g_work;
+    if (g_work) g_work->prev = &w;
+    g_work = &w;
   }
   ~CallMemory() {
     (void)hipStreamSynchronize(s_->stream);  // cleanup: errors are reported where they occur
@@ -626,12 +651,19 @@ void swe_destroy(swe_solver* s) {  // teardown: failures cannot be reported
   if (s->graph) (void)hipGraphExecDestroy(s->graph);
   for (void* p : s->allocs) (void)hipFree(p);
   if (s->dts) (void)hipFree(s->dts);
+  char* work;
   {
     std::lock_guard<std::mutex> lock(g_work_mutex);
-    work_free(&s->work);
+    work = work_take(&s->work);
   }
+  if (work) (void)hipFree(work);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
+}
+
+int swe_release_workspaces(void) {
+  (void)work_release();
+  return SWE_OK;
 }
 
 static int download(swe_solver* s, void* dst, const void* src, size_t bytes) {

@@ -21,7 +21,7 @@ std::mutex m;
 std::map<void*, size_t> held;  // device allocations
 size_t held_bytes = 0;
 std::function<hipError_t()> on_malloc;  // called before an allocation
-std::function<void()> on_free;          // called in every hipFree
+std::function<void(void*)> on_free;     // called in every hipFree
 std::vector<std::function<void()>>* capture = nullptr;
 std::vector<std::vector<std::function<void()>>> graphs;
 const char* fail_launch = nullptr;  // the launch that fails, once
@@ -55,7 +55,7 @@ hipError_t hipMalloc(void** p, size_t n) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
-  if (fake::on_free) fake::on_free();
+  if (fake::on_free) fake::on_free(p);
   {
     std::lock_guard<std::mutex> lock(fake::m);
     if (!fake::held.count(p)) std::abort();
@@ -245,4 +245,130 @@ extern "C" int64_t euler_steps_after_layouts(int layouts, int graph, int runs, i
   for (int64_t i = 0; i < T; ++i)
     if (prim[size_t(3 * i)] != prim[0]) rc = SWE_ERR_ARG;
   return rc == SWE_OK ? int64_t(prim[0]) : -1;
+}
+
+namespace fake {
+std::function<void()> in_stats;  // called by swe_state_stats while it holds its memory
+}
+namespace swe {
+int64_t integrals_blocks(const DevMesh&) { return 1; }
+hipError_t launch_stats(const DevMesh&, const DevState&, double*, double*, hipStream_t) {
+  if (fake::in_stats) fake::in_stats();
+  return hipSuccess;
+}
+}  // namespace swe
+
+namespace {
+
+// a thread's call that waits in a device call until it is let go
+struct Gate {
+  std::mutex m;
+  std::condition_variable cv;
+  bool reached = false, open = false;
+  void wait() {
+    std::unique_lock<std::mutex> l(m);
+    reached = true;
+    cv.notify_all();
+    cv.wait(l, [&] { return open; });
+  }
+  void until_reached() {
+    std::unique_lock<std::mutex> l(m);
+    cv.wait(l, [&] { return reached; });
+  }
+  void let_go() {
+    std::lock_guard<std::mutex> l(m);
+    open = true;
+    cv.notify_all();
+  }
+};
+
+}  // namespace
+
+// While one thread waits in the device (0: hipMalloc of a workspace, 1: hipFree
+// of a destroyed solver's, 2: hipFree of a given-back one), another solver's
+// call on another thread goes through.  1 if it does within 10 s.
+extern "C" int other_solver_goes_on(int kind) {
+  Mesh m(4);
+  swe_solver *a = nullptr, *b = nullptr;
+  if (swe_create(m.t, m.xyz, 1, 2, 0., 0., 0, 0, &a) || swe_create(m.t, m.xyz, 1, 2, 0., 0., 0, 0, &b)) return -1;
+  double out[5];
+  if (kind != 0 && swe_state_stats(a, out)) return -1;
+  Gate gate;
+  std::thread::id slow;
+  std::mutex id;
+  auto hook = [&] {
+    bool here;
+    {
+      std::lock_guard<std::mutex> l(id);
+      here = std::this_thread::get_id() == slow;
+    }
+    if (here) gate.wait();
+  };
+  if (kind == 0) fake::on_malloc = [&] { hook(); return hipSuccess; };
+  else fake::on_free = [&, kept = (void*)a->work.p](void* p) { if (p == kept) hook(); };
+  std::thread ta([&] {
+    {
+      std::lock_guard<std::mutex> l(id);
+      slow = std::this_thread::get_id();
+    }
+    double o[5];
+    if (kind == 0) swe_state_stats(a, o);
+    else if (kind == 1) swe_destroy(a);
+    else swe_release_workspaces();
+  });
+  gate.until_reached();
+  std::atomic<bool> done{false};
+  std::thread tb([&] {
+    double o[5];
+    if (swe_state_stats(b, o) == SWE_OK) done = true;
+  });
+  for (int k = 0; k < 1000 && !done; ++k) std::this_thread::sleep_for(std::chrono::milliseconds(10));
+  const int ok = done ? 1 : 0;
+  gate.let_go();
+  ta.join();
+  tb.join();
+  fake::on_malloc = nullptr;
+  fake::on_free = nullptr;
+  if (kind != 1) swe_destroy(a);
+  swe_destroy(b);
+  return ok;
+}
+
+// Device bytes that n solvers keep after a call each, after they are given back
+// in the middle of one solver's call (which keeps its own), after that, and
+// after another call each
+extern "C" int kept_bytes(int n, int64_t* kept) {
+  Mesh m(4);
+  std::vector<swe_solver*> s(size_t(n), nullptr);
+  for (auto& x : s)
+    if (swe_create(m.t, m.xyz, 1, 2, 0., 0., 0, 0, &x)) return -1;
+  const size_t base = fake::held_bytes;
+  auto call = [&] {
+    double o[5];
+    for (auto x : s)
+      if (swe_state_stats(x, o)) return -1;
+    return 0;
+  };
+  int rc = call();
+  kept[0] = int64_t(fake::held_bytes - base);
+  fake::in_stats = [] { swe_release_workspaces(); };
+  double o[5];
+  rc |= swe_state_stats(s[0], o);
+  fake::in_stats = nullptr;
+  kept[1] = int64_t(fake::held_bytes - base);
+  swe_release_workspaces();
+  kept[2] = int64_t(fake::held_bytes - base);
+  rc |= call();
+  kept[3] = int64_t(fake::held_bytes - base);
+  // an allocation that fails takes them back and is tried again
+  int fails = 1;
+  fake::on_malloc = [&] { return fails-- > 0 ? hipErrorOutOfMemory : hipSuccess; };
+  std::vector<double> wp(size_t(s[0]->V));
+  swe_solver* x = nullptr;
+  rc |= swe_create(m.t, m.xyz, 1, 2, 0., 0., 0, 0, &x);
+  fake::on_malloc = nullptr;
+  if (x) swe_destroy(x);
+  kept[4] = int64_t(fake::held_bytes - base);
+  for (auto y : s) swe_destroy(y);
+  return rc;
 }

@@ -43,3 +43,14 @@ def test_euler_ensembles_after_layout_changes(lib, layouts, graph):
     lib.euler_steps_after_layouts.restype = ctypes.c_int64
     for runs, steps in ((1, 6), (2, 3), (1, 67)):
         assert lib.euler_steps_after_layouts(layouts, graph, runs, ctypes.c_int64(steps)) == runs * steps
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2], ids=["hipMalloc", "hipFree of a destroyed solver", "hipFree of memory given back"])
+def test_solvers_do_not_wait_for_each_others_device_calls(lib, kind):
+    assert lib.other_solver_goes_on(kind) == 1
+
+
+def test_kept_memory_is_given_back(lib):
+    kept = (ctypes.c_int64 * 5)()
+    assert lib.kept_bytes(3, kept) == 0
+    assert kept[0] == 3 * 256 and list(kept)[1:] == [256, 0, 3 * 256, 0]
