@@ -361,7 +361,8 @@ int swe_set_bathymetry(swe_solver* s, const double* z);
 /* Work items per thread of the flux kernel (1, 2 or 4 edges) and of the
  * update kernel (1 or 2 cells); no reference counterpart (the reference is
  * serial).  Results do not depend on the choice, only the speed does.
- * Defaults: 2 and 1. */
+ * Defaults: 2 and 1.  At 2, a flux launch of fewer than 131,072 edges takes
+ * one edge per thread (two would leave parts of the card idle). */
 int swe_set_tuning(swe_solver* s, int flux_items, int update_items);
 int swe_get_tuning(const swe_solver* s, int* flux_items, int* update_items);
 /* Threads per workgroup of the flux and update kernels (256 or 512); no

@@ -615,7 +615,8 @@ class SpaceDisc:
     def set_tuning(self, flux_items=2, update_items=1, flux_block=256, update_block=256):
         """Edges per thread of the flux kernel (1, 2, 4), cells per thread of
         the update kernel (1, 2) and threads per workgroup of either (256,
-        512); results are identical for every choice."""
+        512); results are identical for every choice.  Two edges are
+        taken one by one in launches of fewer than 131,072."""
         _set_tuning(self._h, flux_items, update_items, flux_block, update_block)
 
     def tuning(self):

@@ -33,7 +33,6 @@ struct swe_solver {
   int flux = 1, ws = 2, opts = 0;
   int flux_items = 2, upd_items = 1;  // work items per thread (swe_autotune)
   int flux_block = 256, upd_block = 256;  // threads per workgroup (swe_autotune)
-  bool tuned = false;  // they were set: flux_items_of takes them as they are
   double cor = 0., tau = 0.;
   int64_t T = 0, E = 0, V = 0;
   std::vector<void*> allocs;
@@ -251,12 +250,13 @@ int set_device(swe_solver* s) {
   return SWE_OK;
 }
 
-// Edges per thread of the flux pass.  Untuned, two, whose loads overlap; but
-// one while two would leave SIMDs without a wave (64 lanes x 1,024 SIMDs x 2
-// edges): there a second edge only makes the chain longer.  Us per pass, two /
-// one: 6.1 / 4.7 (1,600 cells), 6.8 / 5.3 (5,000), 7.5 / 5.2 (40,000); 12.4 /
-// 12.9 (250k), 36.2 / 38.2 (1M).
-int flux_items_of(const swe_solver* s) { return !s->tuned && s->M.e1 - s->M.e0 < 64 * 1024 * 2 ? 1 : s->flux_items; }
+// Edges per thread that a flux pass at the setting `items` launches: a setting
+// of two, the default, whose loads overlap, is one while two would leave SIMDs
+// without a wave (64 lanes x 1,024 SIMDs x 2 edges): there a second edge only
+// makes the chain longer.  Us per pass, two / one: 6.1 / 4.7 (1,600 cells),
+// 6.8 / 5.3 (5,000), 7.5 / 5.2 (40,000); 12.4 / 12.9 (250k), 36.2 / 38.2 (1M).
+int flux_items_at(const swe_solver* s, int items) { return items == 2 && s->M.e1 - s->M.e0 < 64 * 1024 * 2 ? 1 : items; }
+int flux_items_of(const swe_solver* s) { return flux_items_at(s, s->flux_items); }
 
 // The fluxes and CFL minimum of the last fused stage, recomputed into W and
 // its r slot from that stage's input (still intact: no stage writes its own
@@ -1285,8 +1285,7 @@ int swe_set_tuning(swe_solver* s, int flux_items, int update_items) {
   if (flux_items != 1 && flux_items != 2 && flux_items != 4)
     return fail(SWE_ERR_ARG, "flux_items must be 1, 2 or 4");
   if (update_items != 1 && update_items != 2) return fail(SWE_ERR_ARG, "update_items must be 1 or 2");
-  if (!s->tuned || s->flux_items != flux_items || s->upd_items != update_items) {
-    s->tuned = true;
+  if (s->flux_items != flux_items || s->upd_items != update_items) {
     s->flux_items = flux_items;
     s->upd_items = update_items;
     if (s->graph) {  // a captured ensemble step holds the old launches
@@ -1366,8 +1365,9 @@ int swe_autotune(swe_solver* s, int reps, int* flux_items, int* update_items, do
   for (int pass = 0; pass < 3 && !rc; ++pass) {
     for (int q = 0; q < 3 && !rc; ++q)
       for (int b = 0; b < 2 && !rc; ++b)
-        rc = timed([&] { return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, rslot, fi[q], bs[b], s->stream); },
-                   t[q][b], pass > 0);
+        rc = timed([&] {
+          return launch_flux(s->M, S, s->W, s->flux, s->ws, s->cor, rslot, flux_items_at(s, fi[q]), bs[b], s->stream);
+        }, t[q][b], pass > 0);
     if (!rc) {
       hipError_t e = launch_drain(s->M, S, s->W, s->opts, s->stream);
       if (e != hipSuccess) rc = dev_fail(e, "drain");

@@ -25,6 +25,7 @@ std::function<void(void*)> on_free;     // called in every hipFree
 std::vector<std::function<void()>>* capture = nullptr;
 std::vector<std::vector<std::function<void()>>> graphs;
 const char* fail_launch = nullptr;  // the launch that fails, once
+int flux_items = 0;                 // edges per thread of the last flux pass
 int64_t listed = 0;                 // cells a reconstruction lists for pass 2
 int64_t list_max = 0;               // the longest the list has been
 
@@ -149,8 +150,9 @@ hipError_t launch_recon2(const DevMesh&, const DevState&, const DevWork&, int, h
   return fake::launch("recon2", [] {});
 }
 hipError_t launch_zero_count(unsigned int* c, hipStream_t) { return fake::launch("zero_count", [=] { *c = 0u; }); }
-hipError_t launch_flux(const DevMesh&, const DevState&, const DevWork&, int, int, double, unsigned long long*, int, int,
-                       hipStream_t, CflMode) {
+hipError_t launch_flux(const DevMesh&, const DevState&, const DevWork&, int, int, double, unsigned long long*, int items,
+                       int, hipStream_t, CflMode) {
+  fake::flux_items = items;
   return fake::launch("flux", [] {});
 }
 hipError_t launch_drain(const DevMesh&, const DevState&, const DevWork&, int, hipStream_t) {
@@ -370,5 +372,32 @@ extern "C" int kept_bytes(int n, int64_t* kept) {
   if (x) swe_destroy(x);
   kept[4] = int64_t(fake::held_bytes - base);
   for (auto y : s) swe_destroy(y);
+  return rc;
+}
+
+// Edges per thread of the flux passes of a solver of n x n squares: as created,
+// after its tuning is read and set again, and after the settings 4, 2 and 1;
+// got: what the getter says after each
+extern "C" int flux_items_launched(int n, int* items, int* got) {
+  Mesh m(n);
+  swe_solver* s = nullptr;
+  if (swe_create(m.t, m.xyz, 1, 2, 0., 0., 0, 0, &s)) return -1;
+  int rc = 0;
+  auto pass = [&](int k) {
+    double r;
+    int u;
+    rc |= swe_compute_fluxes(s, &r) | swe_get_tuning(s, &got[k], &u);
+    items[k] = fake::flux_items;
+    return u;
+  };
+  const int u = pass(0);
+  rc |= swe_set_tuning(s, got[0], u);
+  pass(1);
+  const int set[3] = {4, 2, 1};
+  for (int k = 0; k < 3; ++k) {
+    rc |= swe_set_tuning(s, set[k], u);
+    pass(2 + k);
+  }
+  swe_destroy(s);
   return rc;
 }

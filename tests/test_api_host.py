@@ -54,3 +54,11 @@ def test_kept_memory_is_given_back(lib):
     kept = (ctypes.c_int64 * 5)()
     assert lib.kept_bytes(3, kept) == 0
     assert kept[0] == 3 * 256 and list(kept)[1:] == [256, 0, 3 * 256, 0]
+
+
+@pytest.mark.parametrize("n, two", [(10, 1), (147, 1), (148, 2)])  # 129,948 and 131,720 edges
+def test_the_tuning_that_is_read_can_be_set_again(lib, n, two):
+    items, got = (ctypes.c_int * 5)(), (ctypes.c_int * 5)()
+    assert lib.flux_items_launched(n, items, got) == 0
+    assert list(got) == [2, 2, 4, 2, 1]
+    assert list(items) == [two, two, 4, two, 1]
