@@ -277,7 +277,8 @@ int swe_time_run(swe_solver* s, int scheme, double dt, double cfl, int64_t nstep
 int swe_integrals(swe_solver* s, double* out3, double* per_cell);
 /* Switches the tile kernel off (on = 0) or back on (no reference
  * counterpart).  When on (the default, on meshes whose tiles fit the
- * kernel), every stage whose step size is known before its flux pass (fixed
+ * kernel and whose edges' coordinate differences are zero or of magnitude
+ * 2^-400 .. 2^400; not on periodic ones), every stage whose step size is known before its flux pass (fixed
  * dt; stages 2 and 3 of a CFL step) runs as reconstruction + one fused
  * kernel instead of reconstruction + flux + draining + update, and the first
  * stage of a CFL step as reconstruction + flux + one kernel for the

@@ -521,7 +521,7 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
   // stacked mesh; no edge joins two members)
   if (pe.empty()) {
     StageTables stt;
-    if (plain_geometry(V, px.data(), py.data(), E, ep0.data(), ep1.data()) &&
+    if (plain_geometry(px.data(), py.data(), E, ep0.data(), ep1.data()) &&
         build_stage_tables(T, tp.data(), tt.data(), te.data(), flag.data(), et0.data(), et1.data(), ep0.data(),
                            ep1.data(), stt)) {
       // one block for the tables and the tiles' geometry; the tables of small

@@ -140,13 +140,18 @@ __device__ __forceinline__ double tri_area(const V3& a, const V3& b, const V3& c
   return 0.5 * fabs(ux * vy - vx * uy);
 }
 // Square root and quotients of an edge's geometry whose coordinates the host
-// has checked (plain_geometry): differences and squared length far from the
-// ends of the exponent range, no negative zeros.  There the IEEE square root
-// and division scale nothing and fix nothing up; these are the same
+// has checked (plain_geometry): components of magnitude 2^-400 .. 2^400 or
+// zero, so that the squared length, the quotients and every residual below
+// are normal numbers (2^-906 the smallest bit of one).  There the IEEE square
+// root and division scale nothing and fix nothing up; these are the same
 // roundings without those steps, and with one refined reciprocal for both
 // components of the direction (with the nodes picked from LDS instead of
 // registers: 1701 to 1560 VALU instructions in the fused stage, 111 to 95
-// registers; 238 to 225 us at 4M cells).
+// registers; 238 to 225 us at 4M cells).  The method is Markstein's: Newton
+// steps on the hardware's estimate, then a correction by the residual that a
+// fused multiply-add leaves exact (P. Markstein, Computation of elementary
+// functions on the IBM RISC System/6000 processor, IBM J. Res. Dev. 34, 1990;
+// the square root with Goldschmidt's coupled iteration).
 __device__ __forceinline__ double sqrt_plain(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double s = x * y, h = 0.5 * y;
@@ -162,8 +167,9 @@ __device__ __forceinline__ double rcp_plain(double d) {  // for div_plain only
   return __builtin_fma(__builtin_fma(-d, r, 1.), r, r);
 }
 __device__ __forceinline__ double div_plain(double n, double d, double r) {
+  // the residual with its sign turned, so that a zero n of either sign keeps it
   const double q = n * r;
-  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+  return __builtin_fma(-__builtin_fma(d, q, -n), r, q);
 }
 // Domain::Tang (src/Bathymetry.cpp:69-76): unit (P1 - P0) / L flipped to
 // point outward of the cell with centroid c.  a = P(ep0), b = P(ep1).

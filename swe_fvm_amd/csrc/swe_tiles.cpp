@@ -361,15 +361,12 @@ bool build_stage_tables(int64_t T, const int* tp, const int* tt, const int* te, 
   return true;
 }
 
-bool plain_geometry(int64_t V, const double* px, const double* py, int64_t E, const int* ep0, const int* ep1) {
-  for (int64_t n = 0; n < V; ++n)
-    for (double x : {px[n], py[n]})
-      if (!std::isfinite(x) || (x == 0. && std::signbit(x))) return false;
+bool plain_geometry(const double* px, const double* py, int64_t E, const int* ep0, const int* ep1) {
   const double lo = std::ldexp(1., -400), hi = std::ldexp(1., 400);
   for (int64_t e = 0; e < E; ++e) {
     const double dx = std::fabs(px[ep1[e]] - px[ep0[e]]), dy = std::fabs(py[ep1[e]] - py[ep0[e]]);
     if (dx == 0. && dy == 0.) return false;
-    for (double d : {dx, dy})
+    for (double d : {dx, dy})  // one that is no number is refused here
       if (d != 0. && !(d >= lo && d <= hi)) return false;
   }
   return true;

@@ -95,9 +95,8 @@ bool build_stage_tables(int64_t T, const int* tp, const int* tt, const int* te, 
 
 // whether the edges' geometry needs none of the special cases of the IEEE
 // square root and division (PlainGeometry): every edge's coordinate
-// differences are +0 or of magnitude 2^-400 .. 2^400, not both 0, and no
-// coordinate is a negative zero or not finite
-bool plain_geometry(int64_t V, const double* px, const double* py, int64_t E, const int* ep0, const int* ep1);
+// differences are zero or of magnitude 2^-400 .. 2^400, and not both zero
+bool plain_geometry(const double* px, const double* py, int64_t E, const int* ep0, const int* ep1);
 
 struct DevTiles {
   const TileHead* head;
