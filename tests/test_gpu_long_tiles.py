@@ -17,8 +17,8 @@ def rows():  # 132,480 cells: 517 tiles and a half
     return swe.StructTriangMesh(184, 180, 0.02)
 
 
-def ends():  # 180,000 cells, 44 of them out of order
-    topo = scattered(300, 44)
+def ends():  # 180,000 cells, 73 of them at the end out of order
+    topo = scattered(300, 73)
     return np.array(swe.jittered_mesh(300, 0.25, 8)[0]), topo
 
 

@@ -55,7 +55,7 @@ def scattered(n, k):
 MESHES = {"one square": lambda: swe.StructTriangMesh(1, 1, 0.1)[1], "rows7": lambda: swe.StructTriangMesh(100, 7, 0.1)[1],
           "jittered": lambda: swe.jittered_mesh(61, 0.3, 2)[1], "rows300": lambda: swe.StructTriangMesh(300, 300, 0.1)[1],
           "rows185": lambda: swe.StructTriangMesh(185, 180, 0.1)[1], "jittered300": lambda: swe.jittered_mesh(300, 0.3, 8)[1],
-          "scattered": lambda: scattered(300, 44)}
+          "scattered": lambda: scattered(300, 73)}
 
 
 @pytest.mark.parametrize("mesh", list(MESHES))
@@ -72,3 +72,9 @@ def test_tables_and_lds(lib, mesh):
 def test_morton_ordered_tiles_are_staged_whole(lib):
     _, *lds = check(lib, MESHES["jittered300"]())
     assert lds[0] <= CU // 4 and not lds[2] and not lds[5]
+
+
+@pytest.mark.parametrize("mesh", ["rows300", "rows185", "scattered"])
+def test_long_tiles_leave_the_cells_beyond_the_ring_out(lib, mesh):
+    _, *lds = check(lib, MESHES[mesh]())
+    assert lds[2] and lds[5]
