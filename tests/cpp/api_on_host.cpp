@@ -8,6 +8,7 @@
 #include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <functional>
 #include <map>
 #include <mutex>
@@ -25,6 +26,7 @@ std::function<void(void*)> on_free;     // called in every hipFree
 std::vector<std::function<void()>>* capture = nullptr;
 std::vector<std::vector<std::function<void()>>> graphs;
 const char* fail_launch = nullptr;  // the launch that fails, once
+int launches = 0;                   // kernels so far
 int flux_items = 0;                 // edges per thread of the last flux pass
 int64_t listed = 0;                 // cells a reconstruction lists for pass 2
 int64_t list_max = 0;               // the longest the list has been
@@ -34,6 +36,7 @@ hipError_t launch(const char* name, std::function<void()> f) {
     fail_launch = nullptr;
     return hipErrorLaunchFailure;
   }
+  if (std::strcmp(name, "memcpy") != 0) launches += 1;
   if (capture) capture->push_back(std::move(f));
   else f();
   return hipSuccess;
@@ -400,4 +403,27 @@ extern "C" int flux_items_launched(int n, int* items, int* got) {
   }
   swe_destroy(s);
   return rc;
+}
+
+// A state set and read again on n x n squares in a layout: the launches that
+// it took, or -1 where the state differs or a padding cell is not zero
+extern "C" int launches_of_a_crossing(int n, int layout) {
+  Mesh m(n);
+  swe_solver* s = nullptr;
+  if (swe_create(m.t, m.xyz, 1, 2, 0., 0., 0, 0, &s)) return -1;
+  int rc = swe_set_layout(s, layout);
+  std::vector<double> a(size_t(3 * s->T)), b(a.size());
+  for (size_t k = 0; k < a.size(); ++k) a[k] = double(k + 1);
+  std::memset(s->sbuf[s->cur], 0xff, sizeof(double) * size_t(3 * s->Tpad));
+  const int before = fake::launches;
+  rc |= swe_set_state(s, a.data());
+  const int set = fake::launches - before;
+  const DevState S = state_of(s, s->cur);
+  for (int64_t i = s->T; i < s->Tpad; ++i)
+    if (S.w[S.at(i)] != 0. || S.u[S.at(i)] != 0. || S.v[S.at(i)] != 0.) rc = SWE_ERR_ARG;
+  rc |= swe_get_state(s, b.data());
+  const int all = fake::launches - before;
+  if (a != b || set * 2 != all) rc = SWE_ERR_ARG;
+  swe_destroy(s);
+  return rc ? -1 : all;
 }

@@ -62,3 +62,9 @@ def test_the_tuning_that_is_read_can_be_set_again(lib, n, two):
     assert lib.flux_items_launched(n, items, got) == 0
     assert list(got) == [2, 2, 4, 2, 1]
     assert list(items) == [two, two, 4, two, 1]
+
+
+@pytest.mark.parametrize("layout", [0, 64, 8, 1])
+@pytest.mark.parametrize("n, launches", [(1, 0), (10, 0), (74, 0), (75, 2), (80, 2)])  # 21,904 and 22,500 cells
+def test_small_states_cross_without_a_launch(lib, n, launches, layout):
+    assert lib.launches_of_a_crossing(n, layout) == launches
