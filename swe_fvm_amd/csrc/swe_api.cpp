@@ -570,8 +570,8 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
       s->fused_ok = fused_fits(s->tiles);
     }
   }
-  if ((e = launch_setup_geometry(s->M, G, s->stream)) != hipSuccess) return bail(e, "setup_geometry");
-  if (s->fused_ok && (e = launch_setup_tiles(s->M, s->tiles, s->stream)) != hipSuccess) return bail(e, "setup_tiles");
+  if ((e = launch_setup_geometry(s->M, G, s->fused_ok ? &s->tiles : nullptr, false, s->stream)) != hipSuccess)
+    return bail(e, "setup_geometry");
   if ((e = hipStreamSynchronize(s->stream)) != hipSuccess) return bail(e, "hipStreamSynchronize");
   if (n_inst > 0) {
     s->n_inst = n_inst;
@@ -2017,8 +2017,7 @@ int swe_set_bathymetry(swe_solver* s, const double* z) {
     s->graph = nullptr;
     s->graph_scheme = -1;
   }
-  SWE_CHECK(launch_setup_geometry(s->M, s->G, s->stream), "setup_geometry");
-  if (s->fused_ok) SWE_CHECK(launch_setup_tiles(s->M, s->tiles, s->stream), "setup_tiles");
+  SWE_CHECK(launch_setup_geometry(s->M, s->G, s->fused_ok ? &s->tiles : nullptr, true, s->stream), "setup_geometry");
   SWE_CHECK(hipStreamSynchronize(s->stream), "hipStreamSynchronize");
   return SWE_OK;
 }

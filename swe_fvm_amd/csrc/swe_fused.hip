@@ -390,32 +390,6 @@ __global__ void __launch_bounds__(TH, TH == kTileCells ? SWE_FUSED_MIN_WAVES : T
   out_store<NT>(&O.v[O.at(i)], ov);
 }
 
-// the tiles' copies of the static geometry, one workgroup per tile
-__global__ void __launch_bounds__(256) k_setup_tiles(DevMesh M, DevTiles P) {
-  const int64_t t = blockIdx.x;
-  for (int j = threadIdx.x; j < P.sn; j += 256) {
-    const NodeRec r = M.pn[P.node[t * P.sn + j]];
-    double* const o = P.tnode + t * 3 * P.sn + j;
-    o[0] = r.x;
-    o[P.sn] = r.y;
-    o[2 * P.sn] = r.z;
-  }
-  for (int j = threadIdx.x; j < P.sx; j += 256) {
-    const int x = P.xcell[t * P.sx + j];
-    const CXY c = M.cxy[x];
-    P.txc[2 * (t * P.sx + j)] = c.x;
-    P.txc[2 * (t * P.sx + j) + 1] = c.y;
-    if (j < P.sr) {
-      P.tring[2 * (t * P.sr + j)] = M.bc[x];
-      P.tring[2 * (t * P.sr + j) + 1] = M.area[x];
-    }
-  }
-}
-hipError_t launch_setup_tiles(const DevMesh& M, const DevTiles& P, hipStream_t st) {
-  if (P.ntiles > 0) hipLaunchKernelGGL(k_setup_tiles, dim3((unsigned)P.ntiles), dim3(256), 0, st, M, P);
-  return hipGetLastError();
-}
-
 bool fused_fits(const DevTiles& P) {
   return stage_lds(P, false, true, true) <= kTileMaxLds && stage_lds(P, true, false, true) <= kTileMaxLds;
 }

@@ -69,9 +69,42 @@ __global__ void __launch_bounds__(256) k_setup_cells(DevMesh M, DevGeomOut G) {
   G.cv[i] = CVtx{M.tp[i], M.tp[M.T + i], M.tp[2 * M.T + i], M.cflag[i]};
 }
 
-// min over the edge's two cells of 2 area / length (the flux's CFL length)
-__global__ void __launch_bounds__(256) k_setup_edges(DevMesh M, DevGeomOut G) {
-  int64_t e = global_index();
+// the tiles' copies of the static geometry, one workgroup per tile; z_only:
+// of the heights alone, the rest being there
+__device__ __forceinline__ void setup_tile(const DevMesh& M, const DevGeomOut& G, const DevTiles& P, int64_t t,
+                                           bool z_only) {
+  for (int j = threadIdx.x; j < P.sn; j += kBlock) {
+    const int n = P.node[t * P.sn + j];
+    double* const o = P.tnode + t * 3 * P.sn + j;
+    o[2 * P.sn] = M.pz[n];
+    if (z_only) continue;
+    o[0] = M.px[n];
+    o[P.sn] = M.py[n];
+  }
+  for (int j = threadIdx.x; j < (z_only ? P.sr : P.sx); j += kBlock) {
+    const int x = P.xcell[t * P.sx + j];
+    if (j < P.sr) P.tring[2 * (t * P.sr + j)] = G.bc[x];
+    if (z_only) continue;
+    if (j < P.sr) P.tring[2 * (t * P.sr + j) + 1] = G.area[x];
+    const CXY c = G.cxy[x];
+    P.txc[2 * (t * P.sx + j)] = c.x;
+    P.txc[2 * (t * P.sx + j) + 1] = c.y;
+  }
+}
+
+// min over the edge's two cells of 2 area / length (the flux's CFL length),
+// and in the workgroups after the edges' the tiles: both read what the cells'
+// launch wrote (us per change of bathymetry with a launch of their own that
+// writes every copy / now: 23.6 / 21.5 (288 cells), 41.5 / 38.3 (7,200), 117 /
+// 109 (500,000))
+__global__ void __launch_bounds__(kBlock) k_setup_edges(DevMesh M, DevGeomOut G, DevTiles P, int edge_blocks,
+                                                         int z_only) {
+  if ((int)blockIdx.x >= edge_blocks) {
+    setup_tile(M, G, P, (int64_t)blockIdx.x - edge_blocks, z_only != 0);
+    return;
+  }
+  // logical_block over the edges' workgroups, a multiple of 8
+  const int64_t b = (blockIdx.x & 7) * (edge_blocks >> 3) + (blockIdx.x >> 3), e = b * kBlock + threadIdx.x;
   if (e >= M.E) return;
   const int f = M.et0[e], t = M.et1[e];
   double dm = 0.;
@@ -1253,10 +1286,13 @@ hipError_t scratch_address(double** out) {
 
 // -------------------------------------------------------------- launch --
 
-hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStream_t st) {
+hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, const DevTiles* P, bool z_only, hipStream_t st) {
   hipLaunchKernelGGL(k_setup_nodes, grid_for(M.V), dim3(256), 0, st, M, G);
   hipLaunchKernelGGL(k_setup_cells, grid_for(M.T), dim3(256), 0, st, M, G);
-  hipLaunchKernelGGL(k_setup_edges, grid_for(M.E), dim3(256), 0, st, M, G);
+  const DevTiles tiles = P ? *P : DevTiles{};
+  const unsigned eb = grid_for(M.E).x;
+  hipLaunchKernelGGL(k_setup_edges, dim3(eb + (unsigned)tiles.ntiles), dim3(256), 0, st, M, G, tiles, (int)eb,
+                     z_only ? 1 : 0);
   return hipGetLastError();
 }
 hipError_t launch_recon1(const DevMesh& M, const DevState& S, const DevWork& W, int opts,

@@ -253,7 +253,9 @@ hipError_t launch_relayout(const DevState& S, const DevOut& O, int64_t T, hipStr
 // S's layout; cells [T, Tpad) of O are set to zero
 hipError_t launch_rows_in(const double* rows, const DevOut& O, int64_t T, int64_t Tpad, hipStream_t st);
 hipError_t launch_rows_out(const DevState& S, double* rows, int64_t T, hipStream_t st);
-hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, hipStream_t st);
+// P (may be null): the tiles, whose copies of the geometry are made too;
+// z_only: nothing but the nodes' heights has changed since the last launch
+hipError_t launch_setup_geometry(const DevMesh& M, const DevGeomOut& G, const DevTiles* P, bool z_only, hipStream_t st);
 // zero_count false: W.pw_count is zero already (the stage before cleared it,
 // or launch_slot_counts); r (may be null): set to 1, for the flux pass that
 // follows; P (may be null): by tiles
@@ -334,8 +336,6 @@ hipError_t launch_adjoint_finish(const DevMesh& M, const DevAdj& J, double* zbar
 // of a CFL step's first stage) and are read instead of evaluated.
 // the tiles' data fits the stage kernels' LDS
 bool fused_fits(const DevTiles& P);
-// the tiles' copies of the static geometry, after launch_setup_geometry
-hipError_t launch_setup_tiles(const DevMesh& M, const DevTiles& P, hipStream_t st);
 hipError_t launch_fused(const DevMesh& M, const DevTiles& P, const DevState& S, const DevState& U0,
                         const DevOut& O, const DevWork& W, const StageArgs& A, int flux, int ws, int opts,
                         hipStream_t st, bool store = false, bool from_fluxes = false);

@@ -110,8 +110,7 @@ hipError_t scratch_address(double** p) {
   *p = scratch;
   return hipSuccess;
 }
-hipError_t launch_setup_geometry(const DevMesh&, const DevGeomOut&, hipStream_t) { return hipSuccess; }
-hipError_t launch_setup_tiles(const DevMesh&, const DevTiles&, hipStream_t) { return hipSuccess; }
+hipError_t launch_setup_geometry(const DevMesh&, const DevGeomOut&, const DevTiles*, bool, hipStream_t) { return hipSuccess; }
 hipError_t launch_rows_in(const double* rows, const DevOut& O, int64_t T, int64_t Tpad, hipStream_t) {
   return fake::launch("rows_in", [=] {
     for (int64_t i = 0; i < Tpad; ++i) {
