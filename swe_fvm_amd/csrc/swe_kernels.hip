@@ -1,7 +1,10 @@
 // gfx950 kernels of the explicit finite-volume step.
 //
 // Per stage (Solvers::Euler/SSPRK2/SSPRK3 stage, src/Solvers.cpp:5-59):
-//   k_recon1  per cell  — classification + pass-1 MUSCL (dry / partially wet
+//   k_recon_tile  per tile of the stage kernels (swe_tiles.h), or k_recon1
+//                         per 256 cells where a mesh has no tiles (periodic,
+//                         far from a local order) or they are switched off —
+//                         classification + pass-1 MUSCL (dry / partially wet
 //                         level / full-wet limited plane), stored as
 //                         (w0, gx, gy) per cell: the reference's edge and
 //                         source slots are functions of it and are never
@@ -13,7 +16,11 @@
 //   k_flux    per edge  — HLL/HLLC numerical flux from the two cells' MUSCL
 //                         at the edge midpoint; wave-level + block min of the
 //                         CFL length-to-wavespeed, one 64-bit atomic min per
-//                         block on the positive-double bit pattern.
+//                         block on the positive-double bit pattern, on one of
+//                         eight lines.
+//   k_fused   per tile (swe_fused.hip) — the rest of the stage: with the flux
+//                         pass where the step size is known before it, after
+//                         it otherwise.  Without tiles:
 //   k_drain   per cell  — draining time step from the stage-start state.
 //   k_update  per cell  — fixed-order gather of the three edge fluxes, the
 //                         well-balanced source, SSP-RK stage combination and
@@ -26,7 +33,8 @@
 // Every reduction is either order-independent (max, min) or a fixed-order
 // per-cell gather, so results are deterministic run to run.  Local arrays
 // are only indexed by compile-time constants (unrolled loops) or through
-// register selects, so nothing is placed in scratch or LDS.
+// register selects, so none is placed in scratch; LDS holds the cells, nodes
+// and lists that the reconstruction's workgroups share.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>

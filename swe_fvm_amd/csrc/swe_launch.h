@@ -228,7 +228,8 @@ struct DevTan {
 // the flux pass of 4M cells 11,700 of them, all of its 154 us).  Us per flux
 // pass, one line / eight: 154 / 135 (4M), 16.6 / 12.3 (250k); 1M now 37.1.
 // The readers take the minimum of the lines.  An ensemble's members have an r
-// each, on one line: their workgroups are few.
+// each, 32 bytes apart (four members to a line), not spread: a spread form has
+// not been measured.
 constexpr int kRLines = 8, kRLineWords = 16;
 constexpr int kRSlot = kRLines * kRLineWords;  // words of one flux pass's r
 struct StageArgs {
