@@ -7,6 +7,7 @@ import pytest
 
 import swe_fvm_amd as swe
 from oracle import oracle as O
+from swe_fvm_amd.ensemble import Ensemble
 from tests.test_gpu_tiles import opened, state
 from tests.test_stage_tables_host import scattered
 
@@ -51,3 +52,25 @@ def test_long_tiles_store_the_fluxes_of_the_separate_kernels(opts):
         assert sd.set_fused(fused) == fused
         got.append(sd.adjoint_run(bar, 3, dt=1e-5, checkpoint_every=2)[:2])
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("graph", [True, False])
+@pytest.mark.parametrize("scheme", ["SSPRK2", "SSPRK3"])
+def test_ensembles_of_long_tiles(scheme, graph):
+    # 160,320 cells, 627 tiles while all members run, 470 and fewer once the
+    # first has finished: the launches change form on the way
+    fl = swe.Fluxes.HLLC[swe.Wavespeeds.Einfeldt]
+    doms, prims = [], []
+    for k, (nx, ny, h) in enumerate([(100, 101, 0.08), (100, 99, 0.02), (101, 100, 0.02), (100, 100, 0.03)]):
+        xyz, topo = swe.StructTriangMesh(nx, ny, h)
+        prims.append(state(xyz, topo, 8 + k))
+        doms.append(swe.Domain(xyz, topo))
+    ens = Ensemble(fl, doms, prims)
+    ens.run(scheme, cfl=0.15, t_end=0.03, graph=graph)
+    steps = ens.times()[1]
+    assert steps.min() < steps.max()
+    for k, got in enumerate(ens.states()):
+        one = Ensemble(fl, [doms[k]], [prims[k]])
+        one.run(scheme, cfl=0.15, t_end=0.03, graph=False)
+        assert one.times()[1][0] == steps[k]
+        assert np.array_equal(got, one.states()[0])
