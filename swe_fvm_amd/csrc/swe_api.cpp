@@ -527,10 +527,11 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
                            ep1.data(), stt)) {
       // one block for the tables and the tiles' geometry (an allocation for
       // each made a solver of 40,000 cells 0.4 ms slower to build).  Tables of
-      // up to 1 MB are gathered and cross in one copy (1,600 cells: 0.15 ms
-      // less than one by one); larger ones cross one by one, since touching a
-      // second host copy's pages costs more than the calls (structured mesh
-      // of 40,000 cells, 2.6 MB: 0.56 ms gathered, 0.18 one by one)
+      // up to 2 MB are gathered and cross in one copy (0.15 ms less than one by
+      // one at 1,600 cells, 0.05 at 32,000); larger ones cross one by one,
+      // since touching a second host copy's pages costs more than the calls
+      // (structured mesh of 40,000 cells, 2.6 MB: 0.56 ms gathered, 0.18 one
+      // by one)
       const int64_t nt = stt.ntiles;
       size_t end = 0;
       auto place = [&](size_t bytes) {
@@ -551,7 +552,7 @@ static int create_impl(const Topo& m, const double* xyz, int flux, int wavespeed
       const size_t aring = place(sizeof(double) * size_t(2 * nt * stt.sr));
       char* base = nullptr;
       if ((e = dalloc(s, &base, int64_t(end))) != hipSuccess) return bail(e, "hipMalloc");
-      if (tables <= (size_t(1) << 20)) {
+      if (tables <= (size_t(2) << 20)) {
         std::vector<char> host(tables);
         for (const Part& q : part)
           if (q.bytes) std::memcpy(host.data() + q.at, q.src, q.bytes);
